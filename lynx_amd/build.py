@@ -28,6 +28,7 @@ SOURCES = [
     ("kernels.hip", "hip"),
     ("kernels_scf.hip", "hip"),
     ("kernels_mfma.hip", "hip"),
+    ("kernels_dense.hip", "hip"),
     ("scf.cpp", "hip"),
 ]
 

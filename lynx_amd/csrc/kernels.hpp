@@ -136,6 +136,34 @@ bool gram_f64_fits(const double *A, long lda, const double *B, long ldb);
 size_t rotate_bf16x3_work(int K, int N);
 void rotate_bf16x3(const float *A, long lda, long M, const double *Q, int ldq, int K, int N, void *C, long ldc,
                    bool c_double, void *work, hipStream_t st);
+// Narrow FP64 / complex128 blocks (kernels_dense.hip): units blocks of equal
+// shape (K rows, n columns), at base + u * stride elements of 8 bytes
+// (complex: 16) or at the addresses of a device table; the n x n matrices of
+// consecutive units are contiguous.  narrow_fits: whether n columns of type e
+// are covered (the limits of the kernels' register tiles and LDS).
+constexpr int kNarrowReal = 64, kNarrowComplex = 32;
+struct NarrowBlocks {
+    void *base = nullptr;
+    long stride = 0;
+    void *const *table = nullptr;
+};
+bool narrow_fits(int e, int n);
+int narrow_gram_chunks(int units, long K);
+size_t narrow_gram_work(int e, int n, int units, long K);
+// C = alpha A^H B per unit, Hermitian (B is A with same, else a product whose
+// Hermitian part is taken: its upper triangle is mirrored); aligned: every
+// block starts at a 16-byte boundary.
+void narrow_gram(int e, const NarrowBlocks &A, long lda, const NarrowBlocks &B, long ldb, bool same, bool aligned,
+                 long K, int n, int units, double alpha, void *C, void *work, hipStream_t st);
+// C = A Q per unit; C may be A.
+void narrow_rotate(int e, const NarrowBlocks &A, long lda, const NarrowBlocks &C, long ldc, long K, int n, int units,
+                   const void *Q, hipStream_t st);
+// S -> R^-1 with S = R^H R (zeros below the diagonal); info per unit: the
+// order of the first pivot that is not positive, or 0.
+void narrow_cholesky_inverse(int e, void *S, int n, int units, int *info, hipStream_t st);
+// H -> its eigenvectors, ascending eigenvalues in eval; info per unit: 1 when
+// the iteration did not converge.
+void narrow_eig(int e, void *H, int n, int units, double *eval, int *info, hipStream_t st);
 // Small dense helpers on n x n column-major matrices.
 void hermitian_part(int e, void *H, int n, hipStream_t st);
 void zero_lower(int e, void *H, int n, hipStream_t st);
