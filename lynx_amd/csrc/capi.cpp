@@ -932,6 +932,10 @@ lynx_status lynx_set_grid(lynx_ctx *ctx, int nx, int ny, int nz, const double la
         ctx->has_nl = false;
         ctx->nlh = NonlocalHost{};
         ctx->has_atoms = ctx->has_elec = false;
+        if (ctx->spectral) {
+            HIP_OK(hipStreamSynchronize(ctx->stream));
+            ctx->spectral.reset();
+        }
     });
 }
 
@@ -1938,13 +1942,18 @@ struct lynx_batch {
     struct Unit {
         lynx_ctx *ctx;
         double kpt[3];
-        DevBuf ph64, ph32;     // image phases e^{-i k.R} of this unit's k-point
-        DevBuf work, dx, dy;   // recurrence work block; staging for host buffers
-        DevBuf sy;             // lynx_batch_solve: the filtered block, then H psi, then the rotated block
+        double *ph64 = nullptr;   // image phases e^{-i k.R} of this unit's k-point, in the batch's tables
+        float *ph32 = nullptr;
+        DevBuf dx, dy;         // staging for host buffers
         DevBuf sx32, sy32;     // lynx_batch_solve with the FP32 filter: single-precision copies
         long epoch = -1;       // the context's set-up epoch the phases were built for
     };
     std::vector<Unit> units;
+    // one allocation for all units (an allocation and a free per unit and
+    // kind took 50 ms of a 112-unit SCF run): phase tables; the recurrence
+    // work blocks; lynx_batch_solve's filtered block, then H psi, then the
+    // rotated block
+    DevBuf ph64, ph32, work, sy;
     // plan and graph of the last call; rebuilt when buffers, shapes or dtype change
     std::vector<long> key;
     gpu::BatchPlan *plan = nullptr;
@@ -1970,10 +1979,10 @@ struct lynx_batch {
         gpu::batch_plan_destroy(hplan);
         if (blas) (void)rocblas_destroy_handle(blas);
         for (auto &u : units) {
-            u.ph64.release(); u.ph32.release(); u.work.release(); u.dx.release(); u.dy.release(); u.sy.release();
+            u.dx.release(); u.dy.release();
             u.sx32.release(); u.sy32.release();
         }
-        for (DevBuf *x : {&dmat, &dhs, &dev, &dwork, &dinfo, &dptrs, &dgram}) x->release();
+        for (DevBuf *x : {&dmat, &dhs, &dev, &dwork, &dinfo, &dptrs, &dgram, &ph64, &ph32, &work, &sy}) x->release();
         if (e0) (void)hipEventDestroy(e0);
         if (e1) (void)hipEventDestroy(e1);
         if (stream) (void)hipStreamDestroy(stream);
@@ -1981,22 +1990,35 @@ struct lynx_batch {
 };
 
 namespace {
-// Bloch factors e^{-i k.R_img} of the unit's images at its own k-point,
-// from the context's current projector set-up (rebuilt when a set-up call
-// on the context has changed its images).
-void unit_phases(lynx_batch::Unit &U, hipStream_t st)
+// Bloch factors e^{-i k.R_img} of every unit's images at its own k-point,
+// from the contexts' current projector set-up (rebuilt when a set-up call on
+// a context has changed its images); one table for all units, each unit's
+// part starting at a multiple of 16 image factors.
+void batch_phases(lynx_batch *b)
 {
-    const NonlocalHost &h = U.ctx->nlh;
-    std::vector<double> ph(2 * std::max(1, h.n_img));
-    for (int i = 0; i < h.n_img; ++i) {
-        const double *sh = &h.img_shift[3 * i];
-        const double th = -(U.kpt[0] * sh[0] + U.kpt[1] * sh[1] + U.kpt[2] * sh[2]);
-        ph[2 * i] = std::cos(th);
-        ph[2 * i + 1] = std::sin(th);
+    std::vector<double> ph;
+    std::vector<size_t> off;
+    for (const auto &U : b->units) {
+        const NonlocalHost &h = U.ctx->nlh;
+        off.push_back(ph.size());
+        for (int i = 0; i < h.n_img; ++i) {
+            const double *sh = &h.img_shift[3 * i];
+            const double th = -(U.kpt[0] * sh[0] + U.kpt[1] * sh[1] + U.kpt[2] * sh[2]);
+            ph.push_back(std::cos(th));
+            ph.push_back(std::sin(th));
+        }
+        ph.resize((ph.size() + 32) / 32 * 32);
     }
-    upload(U.ph64, ph, st);
-    upload(U.ph32, std::vector<float>(ph.begin(), ph.end()), st);
-    U.epoch = U.ctx->epoch;
+    const std::vector<float> ph32(ph.begin(), ph.end());
+    upload(b->ph64, ph, b->stream);
+    upload(b->ph32, ph32, b->stream);
+    HIP_OK(hipStreamSynchronize(b->stream));
+    for (size_t u = 0; u < b->units.size(); ++u) {
+        lynx_batch::Unit &U = b->units[u];
+        U.ph64 = b->ph64.as<double>() + off[u];
+        U.ph32 = b->ph32.as<float>() + off[u];
+        U.epoch = U.ctx->epoch;
+    }
 }
 
 template <class F>
@@ -2038,9 +2060,8 @@ lynx_status lynx_batch_create(lynx_batch **out, int nunit, lynx_ctx *const *ctxs
             lynx_batch::Unit &U = b->units[u];
             U.ctx = ctxs[u];
             for (int a = 0; a < 3; ++a) U.kpt[a] = kpts ? kpts[3 * u + a] : 0.0;
-            unit_phases(U, b->stream);
         }
-        HIP_OK(hipStreamSynchronize(b->stream));
+        batch_phases(b);
     });
     if (st != LYNX_OK) {
         delete b;
@@ -2104,15 +2125,23 @@ lynx_status lynx_batch_filter(lynx_batch *b, int dtype, void *const *x, const lo
         // a context whose grid or projectors were set up again since the
         // last call gets new phase tables, and its new set-up epoch and Veff
         // buffers enter the key, so the plan and graph are rebuilt
+        bool stale = false;
+        const lynx_ctx *synced = nullptr;      // units of one context are consecutive in a k-point batch
         for (auto &U : b->units) {
-            HIP_OK(hipStreamSynchronize(U.ctx->stream));
+            if (U.ctx != synced) HIP_OK(hipStreamSynchronize(U.ctx->stream));
+            synced = U.ctx;
             need_gpu_stencil(U.ctx);
             need_veff(U.ctx);
-            if (U.ctx->epoch != U.epoch) unit_phases(U, b->stream);
+            stale = stale || U.ctx->epoch != U.epoch;
         }
+        if (stale) batch_phases(b);
         HIP_OK(hipStreamSynchronize(b->stream));
         std::vector<gpu::BatchUnit> bu(n);
-        std::vector<long> key = {dtype, degree % 2, mem};
+        size_t wtotal = 0;
+        for (int u = 0; u < n; ++u)
+            if (ncol[u] > 0) wtotal += (size_t)padded_ld(b->units[u].ctx->nd) * ncol[u] * es;
+        char *wnext = static_cast<char *>(b->work.get(wtotal));
+        std::vector<long> key = {dtype, degree % 2, mem, (long)(uintptr_t)wnext};
         for (int u = 0; u < n; ++u) {
             lynx_batch::Unit &U = b->units[u];
             lynx_ctx *c = U.ctx;
@@ -2121,7 +2150,8 @@ lynx_status lynx_batch_filter(lynx_batch *b, int dtype, void *const *x, const lo
             const long lx = (ldx && ldx[u]) ? ldx[u] : nd, ly = (ldy && ldy[u]) ? ldy[u] : nd;
             if (lx < nd || ly < nd) fail(LYNX_E_ARG, "leading dimension smaller than Nd");
             const long ldw = padded_ld(nd);
-            void *w = U.work.get((size_t)ldw * ncol[u] * es);
+            void *w = wnext;                   // padded_ld: 64 elements, so each block starts aligned
+            wnext += (size_t)ldw * ncol[u] * es;
             const void *X = x[u];
             void *Y = y[u];
             long lX = lx, lY = ly;
@@ -2139,7 +2169,7 @@ lynx_status lynx_batch_filter(lynx_batch *b, int dtype, void *const *x, const lo
             B.veff = single ? c->veff32.p : c->veff64.p;
             if (c->has_nl) {
                 B.nl = single ? c->nl32 : c->nl64;
-                B.nl.phase = single ? U.ph32.p : U.ph64.p;
+                B.nl.phase = single ? static_cast<const void *>(U.ph32) : U.ph64;
             }
             // odd steps write D1, even steps D2; the last step lands in Y
             void *D1 = (degree % 2 == 1) ? Y : w;
@@ -2157,8 +2187,8 @@ lynx_status lynx_batch_filter(lynx_batch *b, int dtype, void *const *x, const lo
             key.push_back(c->epoch);
             key.push_back(reinterpret_cast<long>(c->veff64.p));
             key.push_back(reinterpret_cast<long>(c->veff32.p));
-            key.push_back(reinterpret_cast<long>(U.ph64.p));
-            key.push_back(reinterpret_cast<long>(U.ph32.p));
+            key.push_back(reinterpret_cast<long>(U.ph64));
+            key.push_back(reinterpret_cast<long>(U.ph32));
         }
         if (key != b->key || !b->plan) {
             if (b->graph) (void)hipGraphExecDestroy(b->graph);
@@ -2250,7 +2280,7 @@ gpu::BatchUnit batch_unit(lynx_batch::Unit &U, int dtype, const void *b0, long l
     B.veff = single ? c->veff32.p : c->veff64.p;
     if (c->has_nl) {
         B.nl = single ? c->nl32 : c->nl64;
-        B.nl.phase = single ? U.ph32.p : U.ph64.p;
+        B.nl.phase = single ? static_cast<const void *>(U.ph32) : U.ph64;
     }
     B.buf[0] = b0; B.buf[1] = b1; B.buf[2] = b2;
     B.ld[0] = l0; B.ld[1] = l1; B.ld[2] = l2;
@@ -2285,6 +2315,7 @@ lynx_status lynx_batch_solve(lynx_batch *b, int dtype, void *const *psi, const l
         const size_t es = gpu::elem_size(dtype);
         std::vector<void *> ys(n);
         std::vector<long> lys(n), lps(n), eoff(n + 1, 0);
+        size_t ytotal = 0;
         for (int u = 0; u < n; ++u) {
             lynx_batch::Unit &U = b->units[u];
             const long nd = U.ctx->nd;
@@ -2293,8 +2324,13 @@ lynx_status lynx_batch_solve(lynx_batch *b, int dtype, void *const *psi, const l
             if (lps[u] < nd) fail(LYNX_E_ARG, "leading dimension smaller than Nd");
             if (ncol[u] > nd) fail(LYNX_E_ARG, "more orbitals than grid points in batch unit " + std::to_string(u));
             lys[u] = padded_ld(nd);
-            ys[u] = U.sy.get((size_t)lys[u] * ncol[u] * es);
             eoff[u + 1] = eoff[u] + ncol[u];
+            ytotal += (size_t)lys[u] * ncol[u] * es;
+        }
+        char *ynext = static_cast<char *>(b->sy.get(ytotal));
+        for (int u = 0; u < n; ++u) {
+            ys[u] = ynext;
+            ynext += (size_t)lys[u] * ncol[u] * es;
         }
         // 1. Y = p(H) psi for every unit (EigenSolver.cpp:558-619); with the
         // FP32 filter on single-precision copies, widened back into Y
@@ -2453,7 +2489,7 @@ lynx_status lynx_batch_solve(lynx_batch *b, int dtype, void *const *psi, const l
                 lynx_batch::Unit &U = b->units[u];
                 bu[u] = batch_unit(U, dtype, psi[u], lps[u], ys[u], lys[u], ys[u], lys[u], ncol[u]);
                 for (long v : {(long)(uintptr_t)psi[u], lps[u], (long)(uintptr_t)ys[u], lys[u], (long)ncol[u],
-                               U.ctx->epoch, (long)(uintptr_t)U.ctx->veff64.p, (long)(uintptr_t)U.ph64.p})
+                               U.ctx->epoch, (long)(uintptr_t)U.ctx->veff64.p, (long)(uintptr_t)U.ph64})
                     key.push_back(v);
             }
             if (key != b->hkey || !b->hplan) {

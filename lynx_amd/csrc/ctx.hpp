@@ -14,6 +14,7 @@
 
 #include <algorithm>
 #include <map>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -144,6 +145,8 @@ struct lynx_ctx {
     long epoch = 0;
     bool use_graphs = true;
 
+    std::shared_ptr<void> spectral;    // FFT plans of the grid (scf.cpp), reset by lynx_set_grid
+
     void *scratch = nullptr;           // this device's scratch array (lynx_h_apply_noalloc)
 
     bool timing = false;
@@ -159,6 +162,7 @@ struct lynx_ctx {
                           &d_cov_gpos, &d_ent_pt, &d_chi64, &d_chi32, &d_gam64, &d_gam32, &d_ph64, &d_ph32,
                           &beta, &wA, &wB, &wC, &lz[0], &lz[1], &lz[2], &s1, &s2, &s3, &gwork, &dvals, &evals,
                           &info, &partials};
+        spectral.reset();
         for (auto &g : graphs)
             if (g.exec) (void)hipGraphExecDestroy(g.exec);
         fcoef.release();

@@ -25,6 +25,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -171,7 +172,25 @@ struct Spectral {
         info = nullptr;
         for (DevBuf *b : {&work, &spec, &sym, &in}) b->release();
     }
+
+    Spectral() = default;
+    Spectral(const Spectral &) = delete;
+    Spectral &operator=(const Spectral &) = delete;
+    ~Spectral() { release(); }
 };
+
+// The transforms of the context's grid, kept by the context until its grid is
+// set again or it is destroyed: planning loads the transforms' code objects,
+// 10 ms for 24^3 or 30^3, which every SCF run of a program would pay again.
+std::shared_ptr<Spectral> spectral_of(lynx_ctx *c)
+{
+    if (!c->spectral) {
+        auto f = std::make_shared<Spectral>();
+        f->init(c->st, c->stream);
+        c->spectral = f;
+    }
+    return std::static_pointer_cast<Spectral>(c->spectral);
+}
 
 }  // namespace
 
@@ -199,7 +218,7 @@ struct lynx_scf {
     DevBuf rhs, ar, af, afo, axo, aX, aF;        // AAR work
     DevBuf mfk, mxkm1, mR, mF, mxw, mfw, mpf, mx, mg;   // mixer state
     DevBuf partials;
-    Spectral fft;                                // LYNX_SOLVE_SPECTRAL
+    std::shared_ptr<Spectral> fft;               // LYNX_SOLVE_SPECTRAL
     int mix_iter = 0;
     std::vector<double> hpart;
 
@@ -218,7 +237,7 @@ struct lynx_scf {
                           &aux, &rhs, &ar, &af, &afo, &axo, &aX, &aF, &mfk, &mxkm1, &mR, &mF, &mxw, &mfw,
                           &mpf, &mx, &mg, &partials};
         if (ctx && ctx->device >= 0) (void)hipSetDevice(ctx->device);
-        fft.release();
+        fft.reset();
         for (DevBuf *x : bufs) x->release();
     }
 };
@@ -330,7 +349,7 @@ void solve_poisson(lynx_scf *S, const double *rho_total)
     gpu::scf_scale(rhs, 4.0 * kPi, n, S->ctx->stream);
     if (S->p.linear_solver == LYNX_SOLVE_SPECTRAL) {
         // zero-mean right side and solution: the q = 0 coefficient is dropped
-        S->fft.solve(rhs, dptr(S->phi), n, 0, 0.0, 0.0, 0.0, S->ctx->stream);
+        S->fft->solve(rhs, dptr(S->phi), n, 0, 0.0, 0.0, 0.0, S->ctx->stream);
         return;
     }
     const double ntot = (double)n;
@@ -487,7 +506,7 @@ void kerker(lynx_scf *S, const double *r, double *z, double amix)
     const double k2 = kKerkerKTF * kKerkerKTF;
     if (S->p.linear_solver == LYNX_SOLVE_SPECTRAL) {
         // z = -amix (-L - idiemac k2) / (L + k2) r
-        S->fft.solve(r, z, n, 1, amix, kKerkerIdiemac * k2, k2, S->ctx->stream);
+        S->fft->solve(r, z, n, 1, amix, kKerkerIdiemac * k2, k2, S->ctx->stream);
         return;
     }
     double *Lf = dptr(S->rhs);
@@ -638,7 +657,7 @@ lynx_status lynx_scf_create(lynx_scf **out, lynx_ctx *ctx, const lynx_scf_params
         S->mR.get((size_t)p->mixing_history * N * sizeof(double));
         S->mF.get((size_t)p->mixing_history * N * sizeof(double));
         S->partials.get((size_t)gpu::kScfPartialBlocks * 40 * sizeof(double));
-        if (p->linear_solver == LYNX_SOLVE_SPECTRAL) S->fft.init(ctx->st, hs);
+        if (p->linear_solver == LYNX_SOLVE_SPECTRAL) S->fft = spectral_of(ctx);
         lynx_scf_eig_params ep{};
         ep.nspin = ns;
         ep.nkpt = p->nkpt;
@@ -767,6 +786,14 @@ lynx_status lynx_scf_run(lynx_scf *S, lynx_scf_result *out)
             for (int k = 0; k < nk; ++k) {
                 const int blk = s * nk + k;
                 blocks[blk] = static_cast<char *>(S->psi.p) + (size_t)blk * S->ldpsi * N * es;
+                if (k > 0) {
+                    // the k-points of a spin share its seed, so they start
+                    // from one drawn block: 112 blocks of 13,824 x 12 complex
+                    // values took 155 ms to draw one by one and upload, and
+                    // take 4 ms as one draw and 111 copies
+                    gpu::copy_cols(dt, blocks[s * nk], S->ldpsi, blocks[blk], S->ldpsi, n, N, hs);
+                    continue;
+                }
                 const lynx_status rs = lynx_randomize(c, dt, blocks[blk], (int)n, (int)S->ldpsi, N,
                                                       (unsigned)(s * 1000 + 1), LYNX_MEM_DEVICE);
                 if (rs != LYNX_OK) fail(rs, std::string("lynx_randomize: ") + lynx_last_error(c));
