@@ -485,11 +485,9 @@ void compute_density(lynx_scf *S, double *out)
     HIP_OK(hipMemcpyAsync(S->w.p, wh.data(), wh.size() * sizeof(double), hipMemcpyHostToDevice, st));
     for (int s = 0; s < ns; ++s) {
         double *rs = ns == 1 ? out : out + (long)(1 + s) * n;
-        for (int k = 0; k < nk; ++k) {
-            const int blk = s * nk + k;
-            const char *P = static_cast<const char *>(S->psi.p) + (size_t)blk * S->ldpsi * N * es;
-            gpu::scf_density(S->cplx, P, S->ldpsi, N, dptr(S->w) + (size_t)blk * N, rs, n, st);
-        }
+        // the spin's k-point blocks lie behind each other: one launch
+        const char *P = static_cast<const char *>(S->psi.p) + (size_t)s * nk * S->ldpsi * N * es;
+        gpu::scf_density(S->cplx, P, S->ldpsi, nk * N, dptr(S->w) + (size_t)s * nk * N, rs, n, st);
     }
     if (ns == 2) {
         dcopy(S, out, out + n, n);
