@@ -3,6 +3,8 @@
 // small helpers.  Launch wrappers at the bottom.
 #include "kernels.hpp"
 #include "common.hpp"
+#include "kernels_points.hpp"
+#include "stencil_common.hpp"
 
 #include <hip/hip_runtime.h>
 #include <algorithm>
@@ -15,119 +17,6 @@ namespace lynx {
 namespace gpu {
 namespace {
 
-// ------------------------------------------------------------ element ops --
-template <class S> struct Tr;
-template <> struct Tr<double> { using A = double; static constexpr bool C = false; };
-template <> struct Tr<float> { using A = float; static constexpr bool C = false; };
-template <> struct Tr<double2> { using A = double; static constexpr bool C = true; };
-template <> struct Tr<float2> { using A = float; static constexpr bool C = true; };
-
-// the FP64 type of each element type (partial sums of single-precision
-// products are added in double precision)
-template <class S> struct Wide { using T = S; };
-template <> struct Wide<float> { using T = double; };
-template <> struct Wide<float2> { using T = double2; };
-__device__ __forceinline__ double widen(double x) { return x; }
-__device__ __forceinline__ double widen(float x) { return (double)x; }
-__device__ __forceinline__ double2 widen(double2 x) { return x; }
-__device__ __forceinline__ double2 widen(float2 x) { return make_double2(x.x, x.y); }
-
-// bfloat16 storage (the filter's BF16 mode): 8-bit mantissa in memory,
-// arithmetic in float.  Conversion to float is exact; from float it rounds
-// to nearest even (finite values).
-struct bf16 {
-    unsigned short b;
-};
-__device__ __forceinline__ float to_compute(bf16 v) { return __uint_as_float((unsigned)v.b << 16); }
-__device__ __forceinline__ float to_compute(float v) { return v; }
-__device__ __forceinline__ double to_compute(double v) { return v; }
-__device__ __forceinline__ double2 to_compute(double2 v) { return v; }
-__device__ __forceinline__ float2 to_compute(float2 v) { return v; }
-template <class T> struct StoreAs;
-template <> struct StoreAs<bf16> {
-    static __device__ __forceinline__ bf16 from(float f)
-    {
-        unsigned u = __float_as_uint(f);
-        u += 0x7fffu + ((u >> 16) & 1u);
-        return bf16{(unsigned short)(u >> 16)};
-    }
-};
-template <> struct StoreAs<float> { static __device__ __forceinline__ float from(float f) { return f; } };
-template <> struct StoreAs<double> { static __device__ __forceinline__ double from(double f) { return f; } };
-template <> struct StoreAs<float2> { static __device__ __forceinline__ float2 from(float2 f) { return f; } };
-template <> struct StoreAs<double2> { static __device__ __forceinline__ double2 from(double2 f) { return f; } };
-
-template <class S> __device__ __forceinline__ S zero();
-template <> __device__ __forceinline__ double zero<double>() { return 0.0; }
-template <> __device__ __forceinline__ float zero<float>() { return 0.0f; }
-template <> __device__ __forceinline__ double2 zero<double2>() { return make_double2(0.0, 0.0); }
-template <> __device__ __forceinline__ float2 zero<float2>() { return make_float2(0.0f, 0.0f); }
-
-__device__ __forceinline__ double add(double a, double b) { return a + b; }
-__device__ __forceinline__ float add(float a, float b) { return a + b; }
-__device__ __forceinline__ double2 add(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
-__device__ __forceinline__ float2 add(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
-
-// scalar * element
-__device__ __forceinline__ double scl(double a, double x) { return a * x; }
-__device__ __forceinline__ float scl(float a, float x) { return a * x; }
-__device__ __forceinline__ double2 scl(double a, double2 x) { return make_double2(a * x.x, a * x.y); }
-__device__ __forceinline__ float2 scl(float a, float2 x) { return make_float2(a * x.x, a * x.y); }
-
-// a * x + y with scalar a
-__device__ __forceinline__ double fm(double a, double x, double y) { return fma(a, x, y); }
-__device__ __forceinline__ float fm(float a, float x, float y) { return fmaf(a, x, y); }
-__device__ __forceinline__ double2 fm(double a, double2 x, double2 y) { return make_double2(fma(a, x.x, y.x), fma(a, x.y, y.y)); }
-__device__ __forceinline__ float2 fm(float a, float2 x, float2 y) { return make_float2(fmaf(a, x.x, y.x), fmaf(a, x.y, y.y)); }
-
-// x * (pr + i pi)
-__device__ __forceinline__ double2 cmul(double2 x, double pr, double pi)
-{
-    return make_double2(x.x * pr - x.y * pi, x.x * pi + x.y * pr);
-}
-__device__ __forceinline__ float2 cmul(float2 x, float pr, float pi)
-{
-    return make_float2(x.x * pr - x.y * pi, x.x * pi + x.y * pr);
-}
-template <class S, class A>
-__device__ __forceinline__ S phased(S v, A pr, A pi)
-{
-    if constexpr (Tr<S>::C) return cmul(v, pr, pi);
-    else return v;
-}
-
-// conj(a) * b and its accumulation
-__device__ __forceinline__ double cfma(double a, double b, double c) { return fma(a, b, c); }
-__device__ __forceinline__ float cfma(float a, float b, float c) { return fmaf(a, b, c); }
-__device__ __forceinline__ double2 cfma(double2 a, double2 b, double2 c)
-{
-    return make_double2(fma(a.x, b.x, fma(a.y, b.y, c.x)), fma(a.x, b.y, fma(-a.y, b.x, c.y)));
-}
-__device__ __forceinline__ float2 cfma(float2 a, float2 b, float2 c)
-{
-    return make_float2(fmaf(a.x, b.x, fmaf(a.y, b.y, c.x)), fmaf(a.x, b.y, fmaf(-a.y, b.x, c.y)));
-}
-// a * b + c (complex)
-__device__ __forceinline__ double mfma_(double a, double b, double c) { return fma(a, b, c); }
-__device__ __forceinline__ float mfma_(float a, float b, float c) { return fmaf(a, b, c); }
-__device__ __forceinline__ double2 mfma_(double2 a, double2 b, double2 c)
-{
-    return make_double2(fma(a.x, b.x, fma(-a.y, b.y, c.x)), fma(a.x, b.y, fma(a.y, b.x, c.y)));
-}
-__device__ __forceinline__ float2 mfma_(float2 a, float2 b, float2 c)
-{
-    return make_float2(fmaf(a.x, b.x, fmaf(-a.y, b.y, c.x)), fmaf(a.x, b.y, fmaf(a.y, b.x, c.y)));
-}
-
-__device__ __forceinline__ double re2(double a) { return a * a; }
-__device__ __forceinline__ double re2(float a) { return double(a) * a; }
-__device__ __forceinline__ double re2(double2 a) { return a.x * a.x + a.y * a.y; }
-__device__ __forceinline__ double re2(float2 a) { return double(a.x) * a.x + double(a.y) * a.y; }
-__device__ __forceinline__ double redot(double a, double b) { return a * b; }
-__device__ __forceinline__ double redot(float a, float b) { return double(a) * b; }
-__device__ __forceinline__ double redot(double2 a, double2 b) { return a.x * b.x + a.y * b.y; }
-__device__ __forceinline__ double redot(float2 a, float2 b) { return double(a.x) * b.x + double(a.y) * b.y; }
-
 // ------------------------------------------------------- fused stencil step --
 // One workgroup owns a band of full x-rows of one column and marches along z
 // over a chunk of planes.  Each thread owns RP points of the band and keeps
@@ -139,44 +28,6 @@ __device__ __forceinline__ double redot(float2 a, float2 b) { return double(a.x)
 // or e^{+i k L} (high side), as the reference halo does
 // (HaloExchange.cpp:104-189).  The work item order puts all bands of one
 // (column, z-chunk) on the same XCD, which dispatches workgroups round-robin.
-template <class A>
-struct StepArgs {
-    const void *x;
-    const void *old;
-    void *out;
-    const A *veff;
-    long ldx, ldo, ldout;
-    int nx, ny, nz, ncol;
-    int tyr, nbands, zch, nzch, nwork;
-    int lpr;            // 16-byte-run kernels: lanes per band row (>= runs per row)
-    A c[3][kMaxR + 1];
-    A a, b, s;
-    A ph[3][2][2];
-    // when set, (a, b, s) are read from this device triple instead (the
-    // filter's steps in a replayed HIP graph take their scalars from a
-    // table uploaded per call)
-    const A *coef = nullptr;
-};
-
-// Per-launch operands of a step (buffers and recurrence scalars), kept
-// apart from the operator record so that a batch can read the record from
-// device memory while these arrive as kernel arguments.
-template <class A>
-struct StepIO {
-    const void *x;
-    const void *old;
-    void *out;
-    long ldx, ldo, ldout;
-    A a, b, s;
-};
-
-template <class A>
-__device__ inline StepIO<A> step_io(const StepArgs<A> &p)
-{
-    if (p.coef) return StepIO<A>{p.x, p.old, p.out, p.ldx, p.ldo, p.ldout, p.coef[0], p.coef[1], p.coef[2]};
-    return StepIO<A>{p.x, p.old, p.out, p.ldx, p.ldo, p.ldout, p.a, p.b, p.s};
-}
-
 // Loads of one z-step, issued one step ahead of their use.
 template <class S, int RP, int HP>
 struct StepLoads {
@@ -186,33 +37,10 @@ struct StepLoads {
     S halo[HP];                  // halo-row values of plane z
 };
 
-// element i of a uniform base pointer, addressed by a 32-bit byte offset so
-// the load can use a scalar base plus a vector offset
-template <class T>
-__device__ __forceinline__ T ld_at(const T *base, unsigned i)
-{
-    return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + i * (unsigned)sizeof(T));
-}
-template <class T>
-__device__ __forceinline__ void st_at(T *base, unsigned i, T v)
-{
-    *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + i * (unsigned)sizeof(T)) = v;
-}
-
-// XCD-aware work order: the hardware hands workgroups to the 8 XCDs round
-// robin, so workgroup b runs on XCD b % 8; mapping it to work item
-// (b % 8) * per + b / 8 gives each XCD a contiguous range of work items.
-__device__ __forceinline__ int xcd_work_item()
-{
-    const int per = gridDim.x >> 3;
-    return (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-}
-
 template <class S, int R, int RP, int NT, int HP, int W>
 __device__ __forceinline__ void stencil_step_body(const StepArgs<typename Tr<S>::A> &p, const StepIO<typename Tr<S>::A> io, const int w)
 {
     using A = typename Tr<S>::A;
-    constexpr bool C = Tr<S>::C;
     constexpr int NR = 2 * R + 1;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     S *lds = reinterpret_cast<S *>(smem_raw);
@@ -264,7 +92,7 @@ __device__ __forceinline__ void stencil_step_body(const StepArgs<typename Tr<S>:
     // halo slots: R rows below and R above the band, wrapped in y
     const int nh = 2 * R * nx;
     unsigned hsrc[HP];
-    int hli[HP], hgh[HP], hgl[HP], hys[HP];
+    int hli[HP], hgh[HP], hgl[HP];
 #pragma unroll
     for (int h = 0; h < HP; ++h) {
         const int t = tid + h * NT;
@@ -273,30 +101,22 @@ __device__ __forceinline__ void stencil_step_body(const StepArgs<typename Tr<S>:
         const int i = tt / nx;
         const int xx = tt - i * nx;
         const int yb = (i < R) ? (i - R) : (rows + i - R);
-        int yg = y0 + yb, ys = 0;
-        if (yg < 0) { yg += ny; ys = 1; }
-        else if (yg >= ny) { yg -= ny; ys = 2; }
+        int yg = y0 + yb;
+        if (yg < 0) yg += ny;
+        else if (yg >= ny) yg -= ny;
         hsrc[h] = v ? yg * nx + xx : 0;
         const int li = (yb + R) * W + xx + R;
         hli[h] = v ? li : dummy;
         hgh[h] = (v && xx < R) ? li + nx : dummy;
         hgl[h] = (v && xx >= nx - R) ? li - nx : dummy;
-        hys[h] = ys;
     }
 
     auto load_plane = [&](int zz, S *dst) {
-        int side = -1;
-        if (zz < 0) { zz += nz; side = 0; }
-        else if (zz >= nz) { zz -= nz; side = 1; }
+        if (zz < 0) zz += nz;
+        else if (zz >= nz) zz -= nz;
         const S *src = X + zz * nxny;
 #pragma unroll
-        for (int r = 0; r < RP; ++r) {
-            S v = ld_at(src, qoff[r]);
-            if constexpr (C) {
-                if (side >= 0) v = phased(v, p.ph[2][side][0], p.ph[2][side][1]);
-            }
-            dst[r] = v;
-        }
+        for (int r = 0; r < RP; ++r) dst[r] = ld_at(src, qoff[r]);
     };
     // every load of plane zs (clamped into the chunk, so the look-ahead past
     // the last plane stays in bounds)
@@ -318,8 +138,8 @@ __device__ __forceinline__ void stencil_step_body(const StepArgs<typename Tr<S>:
     // an element and its wrapped x-ghost copies into the LDS plane
     auto put = [&](S *L, int li, int gh, int gl, S v) {
         L[li] = v;
-        L[gh] = phased(v, p.ph[0][1][0], p.ph[0][1][1]);
-        L[gl] = phased(v, p.ph[0][0][0], p.ph[0][0][1]);
+        L[gh] = v;
+        L[gl] = v;
     };
 
     S ring[RP][NR];
@@ -343,15 +163,7 @@ __device__ __forceinline__ void stencil_step_body(const StepArgs<typename Tr<S>:
             put(L, qli[r], qgh[r], qgl[r], ring[r][R]);
         }
 #pragma unroll
-        for (int h = 0; h < HP; ++h) {
-            S v = cur.halo[h];
-            if constexpr (C) {
-                const A pr = hys[h] == 1 ? p.ph[1][0][0] : (hys[h] == 2 ? p.ph[1][1][0] : A(1));
-                const A pi = hys[h] == 1 ? p.ph[1][0][1] : (hys[h] == 2 ? p.ph[1][1][1] : A(0));
-                v = cmul(v, pr, pi);
-            }
-            put(L, hli[h], hgh[h], hgl[h], v);
-        }
+        for (int h = 0; h < HP; ++h) put(L, hli[h], hgh[h], hgl[h], cur.halo[h]);
         __syncthreads();
         S *Yz = Y + z * nxny;
 #pragma unroll
@@ -394,307 +206,6 @@ __global__ void __launch_bounds__(NT) k_stencil_step(StepArgs<typename Tr<S>::A>
     stencil_step_body<S, R, RP, NT, HP, W>(p, step_io(p), w);
 }
 
-// --------------------------------------- fused stencil, non-orthogonal cell --
-// The non-orthogonal Laplacian adds three mixed terms to the orthogonal one
-// (Hamiltonian.cpp:176-267):
-//   sum_pq cxy[p] d1y[q] (x(+p,+q) - x(+p,-q) - x(-p,+q) + x(-p,-q))  (x,y)
-// and the same for (x,z) with cxz, d1z and (y,z) with cyz, d1z.  Each double
-// sum factors into two one-dimensional antisymmetric sums:
-//   xy: sum_p cxy[p] (g(x+p) - g(x-p)),  g = sum_q d1y[q] (x(y+q) - x(y-q))
-//   xz + yz: sum_q d1z[q] (h(z+q) - h(z-q)),
-//            h = sum_p cxz[p] (x(x+p) - x(x-p)) + cyz[p] (x(y+p) - x(y-p))
-// so a point costs 36 LDS reads and about 60 FMAs instead of 108 four-point
-// groups.  g and h are in-plane quantities: each plane passes through LDS
-// once; g goes back to LDS (with x ghosts) for its x-differences, and h
-// enters the z-difference by forward accumulation: plane f adds its
-// contributions to the 2R+1 pending outputs f-R..f+R held in registers, and
-// output f-R is complete after plane f (the potential term joins the
-// accumulator when the output's own plane passes, so no plane is kept).  A chunk of planes [z0, z1) thus
-// streams planes z0-R .. z1-1+R.  One barrier per plane: the (plane,
-// g-plane) pair is double-buffered and the xy term of plane f is taken one
-// step later, once its g plane is complete.
-// Coefficients are passed factored, D2_a[k] = beta_a w2[k], mixed
-// c_ab[k] = alpha_ab w1[k] and D1_a[k] = w1[k] / h_a, so that the kernel
-// holds 24 scalars instead of 56 (they live in SGPRs).
-template <class A>
-struct NonorthArgs {
-    StepArgs<A> b;
-    A w1[kMaxR + 1];
-    A w2[kMaxR + 1];
-    A beta[3];
-    A axy_hy;            // alpha_xy / h_y
-    A axz, ayz;          // alpha_xz, alpha_yz
-    A ihz;               // 1 / h_z
-};
-
-// PD: planes of global loads in flight ahead of the plane being consumed
-// (1: the next plane; 2: the two next planes, for short-row grids whose
-// steps are latency-bound)
-template <class S, int R, int RP, int NT, int HP, int W, int PD = 1>
-__device__ __forceinline__ void stencil_nonorth_body(const NonorthArgs<typename Tr<S>::A> &q, const StepIO<typename Tr<S>::A> io, const int w)
-{
-    using A = typename Tr<S>::A;
-    constexpr bool C = Tr<S>::C;
-    constexpr int NA = 2 * R + 1;
-    const StepArgs<A> &p = q.b;
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    const int nx = p.nx, ny = p.ny, nz = p.nz;
-    const int dummy = W * (p.tyr + 2 * R) + (int)threadIdx.x;
-    const int plane = W * (p.tyr + 2 * R) + NT;
-    // LDS: two (plane, g-plane) pairs used alternately, so one barrier per
-    // plane suffices: the g of plane f is read one step later
-    S *const lds0 = reinterpret_cast<S *>(smem_raw);
-
-    const int band = w % p.nbands;
-    const int rest = w / p.nbands;
-    const int zc = rest % p.nzch;
-    const int col = rest / p.nzch;
-    const int y0 = band * p.tyr;
-    const int rows = min(p.tyr, ny - y0);
-    const int z0 = zc * p.zch;
-    const int z1 = min(z0 + p.zch, nz);
-    const int nxny = nx * ny;
-
-    const S *__restrict__ X = reinterpret_cast<const S *>(io.x) + (long)col * io.ldx;
-    const S *__restrict__ O = reinterpret_cast<const S *>(io.old) + (long)col * io.ldo;
-    S *__restrict__ Y = reinterpret_cast<S *>(io.out) + (long)col * io.ldout;
-    const bool has_old = io.old != nullptr && io.b != A(0);   // no Y_(k-2) stream without a buffer
-
-    const int tid = threadIdx.x;
-    const int npts = rows * nx;
-    unsigned qoff[RP];
-    int qli[RP], qgh[RP], qgl[RP];
-    bool qv[RP];
-#pragma unroll
-    for (int r = 0; r < RP; ++r) {
-        const int t = tid + r * NT;
-        qv[r] = t < npts;
-        const int tt = qv[r] ? t : 0;
-        const int qy = tt / nx;
-        const int qx = tt - qy * nx;
-        qoff[r] = qv[r] ? (y0 + qy) * nx + qx : 0;
-        const int li = (qy + R) * W + qx + R;
-        qli[r] = qv[r] ? li : dummy;
-        qgh[r] = (qv[r] && qx < R) ? li + nx : dummy;
-        qgl[r] = (qv[r] && qx >= nx - R) ? li - nx : dummy;
-    }
-    const int nh = 2 * R * nx;
-    unsigned hsrc[HP];
-    int hli[HP], hgh[HP], hgl[HP], hys[HP];
-#pragma unroll
-    for (int h = 0; h < HP; ++h) {
-        const int t = tid + h * NT;
-        const bool v = t < nh;
-        const int tt = v ? t : 0;
-        const int i = tt / nx;
-        const int xx = tt - i * nx;
-        const int yb = (i < R) ? (i - R) : (rows + i - R);
-        int yg = y0 + yb, ys = 0;
-        if (yg < 0) { yg += ny; ys = 1; }
-        else if (yg >= ny) { yg -= ny; ys = 2; }
-        hsrc[h] = v ? yg * nx + xx : 0;
-        const int li = (yb + R) * W + xx + R;
-        hli[h] = v ? li : dummy;
-        hgh[h] = (v && xx < R) ? li + nx : dummy;
-        hgl[h] = (v && xx >= nx - R) ? li - nx : dummy;
-        hys[h] = ys;
-    }
-
-    // A workgroup that owns the whole periodic z range marches the nz planes
-    // once (no 2R wrapped planes): the R outputs at each end then lack the
-    // contributions of the planes across the z boundary.  The first R steps
-    // leave the bottom outputs' wrapped part (planes 0..R-1 seen from
-    // nz-R..nz-1, Bloch factor e^{+ikL}) as partial results in Y, the next R
-    // steps store the top outputs 0..R-1 without their wrapped part, and
-    // after the march the ring holds the rest of both, which is added to
-    // those lines of Y (the planes nz-R..nz-1 seen from 0..R-1 with e^{-ikL}).
-    const bool wrapz = p.nzch == 1 && nz >= 2 * R;
-    const int f_end = wrapz ? z1 - 1 : z1 - 1 + R;
-    // every load of plane f (owned points and halo rows, z-wrapped) and of
-    // the output plane f - R (Y_{k-2}, Veff), clamped into range
-    auto issue = [&](int f, StepLoads<S, RP, HP> &L) {
-        f = min(f, f_end);
-        int zz = f;
-        if (zz < 0) zz += nz;
-        else if (zz >= nz) zz -= nz;
-        const S *Xz = X + zz * nxny;
-#pragma unroll
-        for (int r = 0; r < RP; ++r) L.front[r] = ld_at(Xz, qoff[r]);
-#pragma unroll
-        for (int h = 0; h < HP; ++h) L.halo[h] = ld_at(Xz, hsrc[h]);
-        const int zo = max(f - R, z0) * nxny;
-        const int zv = min(max(f, z0), z1 - 1) * nxny;
-#pragma unroll
-        for (int r = 0; r < RP; ++r) {
-            L.old[r] = has_old ? ld_at(O + zo, qoff[r]) : zero<S>();
-            L.v[r] = ld_at(p.veff + zv, qoff[r]);
-        }
-    };
-    auto put = [&](S *L, int li, int gh, int gl, S v) {
-        L[li] = v;
-        L[gh] = phased(v, p.ph[0][1][0], p.ph[0][1][1]);
-        L[gl] = phased(v, p.ph[0][0][0], p.ph[0][0][1]);
-    };
-
-    // acc[j] accumulates -2 (H - s) x at output plane f - R + j; the output's
-    // own plane adds -2 (Veff + s) x there, so H x = -acc / 2 at the end
-    S acc[RP][NA];
-#pragma unroll
-    for (int r = 0; r < RP; ++r)
-#pragma unroll
-        for (int j = 0; j < NA; ++j) acc[r][j] = zero<S>();
-    const A diag = (q.beta[0] + q.beta[1] + q.beta[2]) * q.w2[0];
-
-    int buf = 0;
-    auto step = [&](int f, StepLoads<S, RP, HP> &cur, StepLoads<S, RP, HP> &nxt) {
-        issue(f + PD, nxt);
-        S *LX = lds0 + buf * 2 * plane;
-        S *LG = LX + plane;
-        const S *LGp = lds0 + (buf ^ 1) * 2 * plane + plane;   // g of plane f - 1
-        // z-wrap phase of this plane (uniform)
-        A zr = A(1), zi = A(0);
-        if constexpr (C) {
-            if (f < 0) { zr = p.ph[2][0][0]; zi = p.ph[2][0][1]; }
-            else if (f >= nz) { zr = p.ph[2][1][0]; zi = p.ph[2][1][1]; }
-        }
-        S xf[RP];
-#pragma unroll
-        for (int r = 0; r < RP; ++r) {
-            xf[r] = phased(cur.front[r], zr, zi);
-            put(LX, qli[r], qgh[r], qgl[r], xf[r]);
-        }
-#pragma unroll
-        for (int h = 0; h < HP; ++h) {
-            S v = cur.halo[h];
-            if constexpr (C) {
-                const A pr = hys[h] == 1 ? p.ph[1][0][0] : (hys[h] == 2 ? p.ph[1][1][0] : A(1));
-                const A pi = hys[h] == 1 ? p.ph[1][0][1] : (hys[h] == 2 ? p.ph[1][1][1] : A(0));
-                v = cmul(cmul(v, pr, pi), zr, zi);
-            }
-            put(LX, hli[h], hgh[h], hgl[h], v);
-        }
-        __syncthreads();
-        // xy term of plane f - 1 (its g plane is complete), into output f - 1
-        if (f - 1 >= z0 && f - 1 < z1) {
-#pragma unroll
-            for (int r = 0; r < RP; ++r) {
-                const S *g = LGp + qli[r];
-                S mxy = zero<S>();
-#pragma unroll
-                for (int k = 1; k <= R; ++k) mxy = fm(q.w1[k], add(g[k], scl(A(-1), g[-k])), mxy);
-                acc[r][R - 1] = fm(q.axy_hy, mxy, acc[r][R - 1]);
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        S hz[RP], xzs[RP];
-#pragma unroll
-        for (int r = 0; r < RP; ++r) {
-            const S *c = LX + qli[r];
-            S sx2 = zero<S>(), sy2 = zero<S>(), sx1 = zero<S>(), sy1 = zero<S>();
-            // x then y neighbours; the scheduling barrier keeps the compiler
-            // from hoisting all 24 LDS reads at once (register pressure)
-#pragma unroll
-            for (int k = 1; k <= R; ++k) {
-                const S xp = c[k], xm = c[-k];
-                sx2 = fm(q.w2[k], add(xp, xm), sx2);
-                sx1 = fm(q.w1[k], add(xp, scl(A(-1), xm)), sx1);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int k = 1; k <= R; ++k) {
-                const S yp = c[k * W], ym = c[-k * W];
-                sy2 = fm(q.w2[k], add(yp, ym), sy2);
-                sy1 = fm(q.w1[k], add(yp, scl(A(-1), ym)), sy1);
-            }
-            // in-plane second differences, the potential term (-2 (V + s) x)
-            S a2 = fm(diag - A(2) * (cur.v[r] + io.s), xf[r], scl(q.beta[0], sx2));
-            acc[r][R] = add(acc[r][R], fm(q.beta[1], sy2, a2));
-            hz[r] = scl(q.ihz, fm(q.axz, sx1, scl(q.ayz, sy1)));
-            xzs[r] = scl(q.beta[2], xf[r]);
-            put(LG, qli[r], qgh[r], qgl[r], sy1);
-        }
-        const bool out = f - R >= z0;
-        S *Yz = Y + (f - R) * nxny;
-#pragma unroll
-        for (int r = 0; r < RP; ++r) {
-            // z-terms of plane f for outputs f-R+j, j != R (distance d = R-j)
-#pragma unroll
-            for (int j = 0; j < NA; ++j) {
-                const int d = R - j;
-                if (d != 0) {
-                    const int ad = d > 0 ? d : -d;
-                    acc[r][j] = fm(q.w2[ad], xzs[r], acc[r][j]);
-                    acc[r][j] = fm(d > 0 ? q.w1[ad] : -q.w1[ad], hz[r], acc[r][j]);
-                }
-            }
-            if (out) {
-                S res = scl(A(-0.5) * io.a, acc[r][0]);
-                if (has_old) res = fm(io.b, cur.old[r], res);
-                if (qv[r]) st_at(Yz, qoff[r], res);
-            } else if (wrapz && qv[r]) {
-                // bottom output nz + f - R: its contributions from planes
-                // 0..f, across the boundary
-                const int zo = (nz + f - R) * nxny;
-                S res = scl(A(-0.5) * io.a, phased(acc[r][0], p.ph[2][1][0], p.ph[2][1][1]));
-                if (has_old) res = fm(io.b, ld_at(O + zo, qoff[r]), res);
-                st_at(Y + zo, qoff[r], res);
-            }
-#pragma unroll
-            for (int j = 0; j + 1 < NA; ++j) acc[r][j] = acc[r][j + 1];
-            acc[r][NA - 1] = zero<S>();
-        }
-        buf ^= 1;
-    };
-
-    // a ring of PD + 1 load sets: the step on plane f consumes its set and
-    // refills the one the previous step consumed with plane f + PD
-    StepLoads<S, RP, HP> lring[PD + 1];
-    int f = wrapz ? z0 : z0 - R;
-#pragma unroll
-    for (int d = 0; d < PD; ++d) issue(f + d, lring[d]);
-    for (; f <= f_end; f += PD + 1) {
-#pragma unroll
-        for (int d = 0; d <= PD; ++d)
-            if (f + d <= f_end) step(f + d, lring[d], lring[(d + PD) % (PD + 1)]);
-    }
-    if (!wrapz) return;
-    // the xy term of the last plane (its g plane is complete after a barrier)
-    __syncthreads();
-    {
-        const S *LGp = lds0 + (buf ^ 1) * 2 * plane + plane;
-#pragma unroll
-        for (int r = 0; r < RP; ++r) {
-            const S *g = LGp + qli[r];
-            S mxy = zero<S>();
-#pragma unroll
-            for (int k = 1; k <= R; ++k) mxy = fm(q.w1[k], add(g[k], scl(A(-1), g[-k])), mxy);
-            acc[r][R - 1] = fm(q.axy_hy, mxy, acc[r][R - 1]);
-        }
-    }
-    // ring slot j holds output nz - R + j: the rest of the bottom outputs
-    // (j < R), and for j >= R the planes nz-R..nz-1 seen from top output
-    // j - R across the boundary
-#pragma unroll
-    for (int r = 0; r < RP; ++r) {
-        if (!qv[r]) continue;
-#pragma unroll
-        for (int j = 0; j < 2 * R; ++j) {
-            const int o = j < R ? nz - R + j : j - R;
-            const S c = j < R ? acc[r][j] : phased(acc[r][j], p.ph[2][0][0], p.ph[2][0][1]);
-            S *Yo = Y + o * nxny;
-            st_at(Yo, qoff[r], fm(A(-0.5) * io.a, c, ld_at(Yo, qoff[r])));
-        }
-    }
-}
-
-template <class S, int R, int RP, int NT, int HP, int W>
-__global__ void __launch_bounds__(NT) k_stencil_nonorth(NonorthArgs<typename Tr<S>::A> q)
-{
-    const int w = xcd_work_item();
-    if (w >= q.b.nwork) return;
-    stencil_nonorth_body<S, R, RP, NT, HP, W>(q, step_io(q.b), w);
-}
-
 // ------------------------------------------------ fused stencil, 16-B runs --
 // Same step as k_stencil_step for real element types, with each thread owning
 // runs of VW consecutive x points: 16-byte runs (two doubles, four floats),
@@ -704,49 +215,6 @@ __global__ void __launch_bounds__(NT) k_stencil_nonorth(NonorthArgs<typename Tr<
 // read per offset.  This cuts the LDS instructions per point by about 2.5x
 // and makes every global access a dwordx4 (dwordx2).  Requires nx % VW == 0
 // and columns aligned to the run size.
-template <class S, int VW>
-struct alignas(sizeof(S) * VW) VRun {
-    S v[VW];
-};
-
-template <class S, int VW>
-__device__ __forceinline__ VRun<S, VW> vzero()
-{
-    VRun<S, VW> r;
-#pragma unroll
-    for (int e = 0; e < VW; ++e) r.v[e] = S(0);
-    return r;
-}
-
-template <int VW, class S>
-__device__ __forceinline__ VRun<S, VW> vld(const S *base, unsigned i)
-{
-    return *reinterpret_cast<const VRun<S, VW> *>(reinterpret_cast<const char *>(base) + i * (unsigned)sizeof(S));
-}
-
-// a run of storage type T loaded into compute type S, and stored back
-template <int VW, class S, class T>
-__device__ __forceinline__ VRun<S, VW> vldc(const T *base, unsigned i)
-{
-    if constexpr (std::is_same<S, T>::value) {
-        return vld<VW>(base, i);
-    } else {
-        const VRun<T, VW> t = vld<VW>(base, i);
-        VRun<S, VW> r;
-#pragma unroll
-        for (int e = 0; e < VW; ++e) r.v[e] = to_compute(t.v[e]);
-        return r;
-    }
-}
-template <int VW, class S, class T>
-__device__ __forceinline__ void vstc(T *base, unsigned i, const VRun<S, VW> &v)
-{
-    VRun<T, VW> t;
-#pragma unroll
-    for (int e = 0; e < VW; ++e) t.v[e] = StoreAs<T>::from(v.v[e]);
-    *reinterpret_cast<VRun<T, VW> *>(reinterpret_cast<char *>(base) + i * (unsigned)sizeof(T)) = t;
-}
-
 template <class S, int VW, int RV, int HP>
 struct VecLoads {
     VRun<S, VW> front[RV];
@@ -1169,13 +637,6 @@ __global__ void __launch_bounds__(NT) k_stencil_vacc(StepArgs<S> p)
 // interleaved runs of the atom's sphere points (all images); each lane
 // accumulates npm projections, then a wave reduction, and the four wave sums
 // are added in a fixed order through LDS (deterministic, no atomics).
-template <class A>
-struct NlArgs {
-    const int *atom_pt_off, *pt_gpos, *pt_img, *pt_atom, *cov_off, *cov_gpos, *ent_pt;
-    const A *chi, *gamma, *phase;
-    int n_atom, n_cov, npm;
-};
-
 // SPLIT = false: one wave per column (four columns per workgroup, index c
 // is the column group); SPLIT = true: the four waves share one column (c)
 // and split the points, for atoms with many sphere points.
@@ -1350,53 +811,25 @@ __global__ void __launch_bounds__(256) k_nl_scatter_mc(NlArgs<typename Tr<S>::A>
 // kernel covers every unit.  Work items of a unit are contiguous, so the
 // XCD-aware order keeps a unit's bands on one XCD; a table maps each work
 // item to its unit.
-template <class A>
-struct BatchRec {
-    NonorthArgs<A> q;           // operator of the unit; pointers and a, b, s set per step
-    const void *buf[4];         // X, D1, D2, none
-    long ld[4];
-    int item0;                  // first stencil work item
-    int g_item0, s_item0;       // first gather / scatter block
-    int ncol;
-    int s_cpw;                  // scatter columns per wave
-    long beta_off;              // first beta element of the unit
-    NlArgs<A> nl;
-    // gather by parts (units with large spheres): sphere point ranges
-    // [pb, pe) of at most kGatherPartPts points of one atom, the first part
-    // of each atom (n_atom + 1), and the unit's first partial sum
-    const int2 *parts;
-    const int *atom_part;
-    int nparts;
-    int r_item0;                // first reduction block
-    long part_off;
-};
-
-// KIND: 0 orthogonal (scalar body), 1 non-orthogonal, 2 orthogonal with
-// 16-byte runs and row-aligned lanes (real types, RP runs per thread; the
-// forward-accumulation body with loads two planes ahead), 3 the same with
-// 8-byte runs of two floats
+// KIND: 0 real orthogonal units, scalar body; 2 the same with 16-byte runs
+// and row-aligned lanes (RP runs per thread; the forward-accumulation body
+// with loads two planes ahead); 3 the same with 8-byte runs of two floats.
+// Complex and non-orthogonal units (kind 1) run in points_batch.
 template <class S, int R, int RP, int NT, int HP, int W, int KIND>
-__global__ void __launch_bounds__(NT) k_stencil_batch(const BatchRec<typename Tr<S>::A> *__restrict__ recs,
+__global__ void __launch_bounds__(NT) k_stencil_batch(const BatchRec<S> *__restrict__ recs,
                                                       const int *__restrict__ item_unit, int nitems,
-                                                      const typename Tr<S>::A *__restrict__ coef, int ix,
-                                                      int iold, int iout)
+                                                      const S *__restrict__ coef, int ix, int iold, int iout)
 {
-    using A = typename Tr<S>::A;
     const int w = xcd_work_item();
     if (w >= nitems) return;
     const int u = item_unit[w];
-    const BatchRec<A> &r = recs[u];
-    const StepIO<A> io{r.buf[ix], r.buf[iold], const_cast<void *>(r.buf[iout]), r.ld[ix], r.ld[iold], r.ld[iout],
+    const BatchRec<S> &r = recs[u];
+    const StepIO<S> io{r.buf[ix], r.buf[iold], const_cast<void *>(r.buf[iout]), r.ld[ix], r.ld[iold], r.ld[iout],
                        coef[3 * u], coef[3 * u + 1], coef[3 * u + 2]};
-    if constexpr (KIND == 1) {
-        // batched units are small grids: two planes of loads in flight
-        stencil_nonorth_body<S, R, RP, NT, HP, W, 2>(r.q, io, w - r.item0);
-    } else if constexpr (KIND == 2 || KIND == 3) {
-        if constexpr (!Tr<S>::C)
-            stencil_vacc_body<S, R, RP, NT, HP, W, 2, KIND == 3 ? 2 : int(16 / sizeof(S))>(r.q.b, io, w - r.item0);
-    } else {
+    if constexpr (KIND == 2 || KIND == 3)
+        stencil_vacc_body<S, R, RP, NT, HP, W, 2, KIND == 3 ? 2 : int(16 / sizeof(S))>(r.q.b, io, w - r.item0);
+    else
         stencil_step_body<S, R, RP, NT, HP, W>(r.q.b, io, w - r.item0);
-    }
 }
 
 // Batched gather of units whose atoms have small spheres: one workgroup per
@@ -1785,68 +1218,6 @@ void launch_step_rp(const StencilGeom &g, const void *x, long ldx, const void *o
     }
 }
 
-template <class S, int RP, int NT>
-void launch_step_nonorth(const StencilGeom &g, const void *x, long ldx, const void *old, long ldo, void *out,
-                         long ldout, const void *veff, int ncol, double a, double b, double s, int nzch,
-                         hipStream_t st, const void *coef = nullptr)
-{
-    using A = typename Tr<S>::A;
-    constexpr int HS = NT >= 512 ? 2 : 3;
-    constexpr int HB = NT >= 512 ? 3 : 6;
-    const long pts = (long)NT * RP;
-    if (!step_rows_fit<S>(g.nx, NT, RP, true))
-        fail(8, "grid rows longer than the fused stencil kernel's tile are not supported");
-    NonorthArgs<A> q;
-    StepArgs<A> &p = q.b;
-    p.x = x; p.old = old; p.out = out; p.veff = static_cast<const A *>(veff);
-    p.ldx = ldx; p.ldo = ldo; p.ldout = ldout;
-    p.nx = g.nx; p.ny = g.ny; p.nz = g.nz; p.ncol = ncol;
-    // short rows: a 40-point pitch, so more workgroups fit a CU
-    const int pitch = g.nx + 2 * kMaxR <= 40 ? 40 : tile_pitch(g.nx);
-    const int max_rows = nonorth_max_rows<S>(pitch, NT);
-    int nb = (int)(((long)g.nx * g.ny + pts - 1) / pts);
-    nb = std::max(1, std::min(nb, g.ny));
-    p.tyr = (g.ny + nb - 1) / nb;
-    while ((long)p.tyr * g.nx > pts || p.tyr > max_rows) { ++nb; p.tyr = (g.ny + nb - 1) / nb; }
-    p.nbands = (g.ny + p.tyr - 1) / p.tyr;
-    nzch = std::max(1, std::min(nzch, g.nz));
-    p.zch = (g.nz + nzch - 1) / nzch;
-    p.nzch = (g.nz + p.zch - 1) / p.zch;
-    p.nwork = p.nbands * p.nzch * ncol;
-    for (int ax = 0; ax < 3; ++ax)
-        for (int k = 0; k <= kMaxR; ++k) p.c[ax][k] = (A)g.c[ax][k];
-    for (int k = 0; k <= kMaxR; ++k) {
-        q.w1[k] = (A)g.w1[k];
-        q.w2[k] = (A)g.w2[k];
-    }
-    for (int ax = 0; ax < 3; ++ax) q.beta[ax] = (A)g.beta[ax];
-    q.axy_hy = (A)(g.alpha[0] / g.h[1]);
-    q.axz = (A)g.alpha[1];
-    q.ayz = (A)g.alpha[2];
-    q.ihz = (A)(1.0 / g.h[2]);
-    p.a = (A)a; p.b = (A)b; p.s = (A)s;
-    p.coef = static_cast<const A *>(coef);
-    for (int ax = 0; ax < 3; ++ax)
-        for (int sd = 0; sd < 2; ++sd)
-            for (int k = 0; k < 2; ++k) p.ph[ax][sd][k] = (A)g.phase[ax][sd][k];
-    const int blocks = ((p.nwork + 7) / 8) * 8;
-    const size_t shm = 4 * sizeof(S) * ((size_t)pitch * (p.tyr + 2 * kMaxR) + NT);
-    const bool small_halo = 2 * kMaxR * g.nx <= NT * HS;
-    if (pitch == 40) {
-        if (small_halo) hipLaunchKernelGGL((k_stencil_nonorth<S, kMaxR, RP, NT, HS, 40>), dim3(blocks), dim3(NT), shm, st, q);
-        else hipLaunchKernelGGL((k_stencil_nonorth<S, kMaxR, RP, NT, HB, 40>), dim3(blocks), dim3(NT), shm, st, q);
-    } else if (pitch == 64) {
-        if (small_halo) hipLaunchKernelGGL((k_stencil_nonorth<S, kMaxR, RP, NT, HS, 64>), dim3(blocks), dim3(NT), shm, st, q);
-        else hipLaunchKernelGGL((k_stencil_nonorth<S, kMaxR, RP, NT, HB, 64>), dim3(blocks), dim3(NT), shm, st, q);
-    } else if (pitch == 128) {
-        if (small_halo) hipLaunchKernelGGL((k_stencil_nonorth<S, kMaxR, RP, NT, HS, 128>), dim3(blocks), dim3(NT), shm, st, q);
-        else hipLaunchKernelGGL((k_stencil_nonorth<S, kMaxR, RP, NT, HB, 128>), dim3(blocks), dim3(NT), shm, st, q);
-    } else if constexpr (NT >= 512 && sizeof(S) <= 8) {
-        // long rows; complex128 planes of pitch 256 do not fit the LDS (step_rows_fit)
-        hipLaunchKernelGGL((k_stencil_nonorth<S, kMaxR, RP, NT, kLongHalo, 256>), dim3(blocks), dim3(NT), shm, st, q);
-    }
-}
-
 // run width of the vector stencil for rows of nx points: 16-byte runs, else
 // (floats) 8-byte runs, else 0 (no vector form)
 template <class S>
@@ -2008,35 +1379,33 @@ void stencil_step(int e, const StencilGeom &g, const void *x, long ldx, const vo
     dispatch(e, [&](auto t) {
         using S = decltype(t);
         constexpr int B = base_rp<S>();
-        if (!g.orth) {
-            // non-orthogonal cells: 2R+1 accumulators per point, so a quarter
-            // of the orthogonal kernel's points per thread (8 B per thread for
-            // points_div 1, half that for 2, at least one point)
-            constexpr int B2 = B / 4 > 0 ? B / 4 : 1;
-            constexpr int B4 = B / 8 > 0 ? B / 8 : 1;
-            if (cfg.nt >= 512) {
-                if (cfg.rp_div >= 2) launch_step_nonorth<S, B4, 512>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
-                else launch_step_nonorth<S, B2, 512>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
-            } else {
-                if (cfg.rp_div >= 2) launch_step_nonorth<S, B4, 256>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
-                else launch_step_nonorth<S, B2, 256>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
-            }
+        if (!g.orth || Tr<S>::C) {
+            // one point per thread (stencil_points.hpp); the rows each of the
+            // four shapes takes are those of its tile, points per thread
+            // included, as the tuner lists them
+            const int nt = cfg.nt >= 512 ? 512 : 256;
+            const int rp = std::max(1, (g.orth ? B : B / 4) / (cfg.rp_div >= 2 ? 2 : 1));
+            PointShape sh;
+            if (!step_rows_fit<S>(g.nx, nt, rp, !g.orth) ||
+                !point_shape(e, g, cfg.rp_div >= 2 ? nt / 4 * 3 : nt, cfg.nzch, sh))
+                fail(8, "grid rows longer than the fused stencil kernel's tile are not supported");
+            points_step(e, g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, sh, st, coef);
             return;
         }
         if constexpr (!Tr<S>::C) {
             if (cfg.vec && launch_vec_modes<S, S>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg, st, coef))
                 return;
-        }
-        if (cfg.nt >= 512) {
-            if (cfg.rp_div >= 2)
-                launch_step_rp<S, B / 2, 512>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
-            else
-                launch_step_rp<S, B, 512>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
-        } else {
-            if (cfg.rp_div >= 2)
-                launch_step_rp<S, B / 2, 256>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
-            else
-                launch_step_rp<S, B, 256>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
+            if (cfg.nt >= 512) {
+                if (cfg.rp_div >= 2)
+                    launch_step_rp<S, B / 2, 512>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
+                else
+                    launch_step_rp<S, B, 512>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
+            } else {
+                if (cfg.rp_div >= 2)
+                    launch_step_rp<S, B / 2, 256>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
+                else
+                    launch_step_rp<S, B, 256>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
+            }
         }
     });
 }
@@ -2112,13 +1481,15 @@ struct BatchPlan {
     int e = 0, n = 0;
     void *recs = nullptr;
     struct SGroup {
-        int kind = 0;             // 0 orthogonal, 1 non-orthogonal, 2 / 3 orthogonal 16- / 8-byte runs
+        int kind = 0;             // 0 real orthogonal, 1 complex or non-orthogonal, 2 / 3 real orthogonal 16- / 8-byte runs
         int W = 64;
         int *items = nullptr;
         int nitems = 0;
         int max_tyr = 0;
         bool small_halo = true;   // fewer halo slots per thread suffice for every unit of the group
-        int nt = 256;             // threads per workgroup (192 for short-row non-orthogonal groups, 512 for long rows)
+        int nt = 256;             // threads per workgroup (512 for long rows)
+        bool nonorth = false;     // kind 1: cell, and launch shape of its units (rows per band differ)
+        PointShape shape;
     };
     struct NGroup {
         int npm = 8;
@@ -2153,15 +1524,10 @@ T *dev_upload(const std::vector<T> &v, hipStream_t st)
 
 // points per thread of the batched stencil shapes (256 threads per group)
 template <class S> constexpr int batch_rp_orth() { return base_rp<S>() / 2 > 0 ? base_rp<S>() / 2 : 1; }
-template <class S> constexpr int batch_rp_nonorth() { return base_rp<S>() / 4 > 0 ? base_rp<S>() / 4 : 1; }
 constexpr int kBatchNT = 256;
 // runs per thread of the batched run-vector kinds (two, for taller bands
 // and less halo, ran slower: more registers, fewer waves)
 constexpr int kBatchRuns = 1;
-// LDS row pitch of batched non-orthogonal units with rows of at most
-// 40 - 2R points
-constexpr int kShortNonorthPitch = 40;
-
 template <class S>
 void build_batch(BatchPlan *P, const BatchUnit *units, int n, hipStream_t st)
 {
@@ -2170,37 +1536,26 @@ void build_batch(BatchPlan *P, const BatchUnit *units, int n, hipStream_t st)
     // stencil groups by (orth, pitch, threads), nonlocal groups by npm
     std::vector<int> sgi(n), ngi(n, -1);
     std::vector<int> kind(n), ntu(n, kBatchNT);
-    // lanes of a non-orthogonal tile with nt threads that hold a point
-    auto nonorth_fill = [&](const StencilGeom &g, int nt, int W) {
-        const long pts = (long)nt * batch_rp_nonorth<S>();
-        const int max_rows = nonorth_max_rows<S>(W, nt);
-        if (max_rows < 1 || g.nx > pts) return 0.0;
-        int nb = (int)std::max<long>(1, std::min<long>(((long)g.nx * g.ny + pts - 1) / pts, g.ny));
-        int tyr = (g.ny + nb - 1) / nb;
-        while ((long)tyr * g.nx > pts || tyr > max_rows) { ++nb; tyr = (g.ny + nb - 1) / nb; }
-        nb = (g.ny + tyr - 1) / tyr;
-        return (double)g.nx * g.ny / ((double)nb * pts);
-    };
+    std::vector<PointShape> shape(n);
     for (int u = 0; u < n; ++u) {
         const StencilGeom &g = units[u].g;
         if (g.nx + 2 * kMaxR > 256) fail(8, "grid rows longer than the fused stencil kernel's tile are not supported");
-        kind[u] = g.orth ? 0 : 1;
+        kind[u] = g.orth && !Tr<S>::C ? 0 : 1;
         int W = tile_pitch(g.nx);
-        if (!g.orth && g.nx + 2 * kMaxR <= kShortNonorthPitch) W = kShortNonorthPitch;
         bool sh = 2 * kMaxR * g.nx <= kBatchNT * 3;
-        if (W == 256) {
+        if (kind[u] == 1) {
+            if (!g.orth && W == 256 && sizeof(S) > 8)
+                fail(8, "complex128 non-orthogonal grids with rows over 116 points are not supported");
+            if (!point_shape_batch(P->e, g, shape[u]))
+                fail(8, "grid rows longer than the batched stencil kernel's tile are not supported");
+            W = shape[u].pitch;
+            ntu[u] = shape[u].nt;
+            sh = true;
+        } else if (W == 256) {
             // long rows: 512 threads, a 256-point pitch and kLongHalo halo
             // slots per thread, scalar bodies (no vector runs)
-            if (!g.orth && sizeof(S) > 8)
-                fail(8, "complex128 non-orthogonal grids with rows over 116 points are not supported");
             ntu[u] = 512;
             sh = false;
-        } else if (!g.orth && 2 * kMaxR * g.nx <= 192 * 2 && nonorth_fill(g, 192, W) > nonorth_fill(g, kBatchNT, W)) {
-            // short non-orthogonal rows: 192 threads (two halo slots each)
-            // when they leave fewer lanes idle than 256, e.g. 8 rows of 24
-            // points
-            ntu[u] = 192;
-            sh = true;
         }
         if constexpr (!Tr<S>::C) {
             // kind 2: 16-byte runs; kind 3: 8-byte runs of two floats for
@@ -2226,13 +1581,16 @@ void build_batch(BatchPlan *P, const BatchUnit *units, int n, hipStream_t st)
         }
         int k = -1;
         for (size_t i = 0; i < P->sg.size(); ++i)
-            if (P->sg[i].kind == kind[u] && P->sg[i].W == W && P->sg[i].small_halo == sh && P->sg[i].nt == ntu[u])
+            if (P->sg[i].kind == kind[u] && P->sg[i].W == W && P->sg[i].small_halo == sh && P->sg[i].nt == ntu[u] &&
+                (kind[u] != 1 || (P->sg[i].nonorth == !g.orth && P->sg[i].shape.hp == shape[u].hp &&
+                                  P->sg[i].shape.wrapz == shape[u].wrapz)))
                 k = (int)i;
         if (k < 0) {
-            P->sg.push_back({kind[u], W, nullptr, 0, 0, sh, ntu[u]});
+            P->sg.push_back({kind[u], W, nullptr, 0, 0, sh, ntu[u], !g.orth, shape[u]});
             k = (int)P->sg.size() - 1;
         }
         sgi[u] = k;
+        P->sg[k].shape.lds = std::max(P->sg[k].shape.lds, shape[u].lds);
         if (units[u].nl.n_atom > 0 && units[u].nl.n_pts > 0) {
             const bool split = units[u].nl.max_atom_pts > kGatherSplitPts;
             int j = -1;
@@ -2259,9 +1617,9 @@ void build_batch(BatchPlan *P, const BatchUnit *units, int n, hipStream_t st)
         const BatchUnit &U = units[u];
         const StencilGeom &g = U.g;
         BatchRec<A> &r = recs[u];
-        NonorthArgs<A> &q = r.q;
-        StepArgs<A> &p = q.b;
-        p.nx = g.nx; p.ny = g.ny; p.nz = g.nz; p.ncol = U.ncol;
+        r.q = operator_args<A>(g);
+        StepArgs<A> &p = r.q.b;
+        p.ncol = U.ncol;
         if (kind[u] == 2 || kind[u] == 3) {
             // kBatchRuns runs per thread, band rows at lane multiples of 16
             const int VW = kind[u] == 3 ? 2 : int(16 / sizeof(S));
@@ -2269,15 +1627,17 @@ void build_batch(BatchPlan *P, const BatchUnit *units, int n, hipStream_t st)
             const int rpb = kBatchRuns * kBatchNT / p.lpr;
             const int nb = (g.ny + rpb - 1) / rpb;
             p.tyr = (g.ny + nb - 1) / nb;
+        } else if (kind[u] == 1) {
+            p.lpr = 0;
+            p.tyr = shape[u].tyr;
         } else {
             const int nt = ntu[u];
-            const long pts = (long)nt * (g.orth ? batch_rp_orth<S>() : batch_rp_nonorth<S>());
-            const int hslots = nt == 512 ? kLongHalo : (nt == kBatchNT ? 6 : 2);
+            const long pts = (long)nt * batch_rp_orth<S>();
+            const int hslots = nt == 512 ? kLongHalo : 6;
             if (g.nx > pts || 2 * kMaxR * g.nx > nt * hslots)
                 fail(8, "grid rows longer than the batched stencil kernel's tile are not supported");
             p.lpr = 0;
-            const int pitch = P->sg[sgi[u]].W;
-            const int max_rows = g.orth ? step_max_rows<S>(pitch, nt) : nonorth_max_rows<S>(pitch, nt);
+            const int max_rows = step_max_rows<S>(P->sg[sgi[u]].W, nt);
             if (max_rows < 1) fail(8, "grid rows longer than the batched stencil kernel's tile are not supported");
             int nb = (int)(((long)g.nx * g.ny + pts - 1) / pts);
             nb = std::max(1, std::min(nb, g.ny));
@@ -2289,20 +1649,6 @@ void build_batch(BatchPlan *P, const BatchUnit *units, int n, hipStream_t st)
         p.nzch = 1;
         p.nwork = p.nbands * U.ncol;
         p.veff = static_cast<const A *>(U.veff);
-        for (int ax = 0; ax < 3; ++ax)
-            for (int k = 0; k <= kMaxR; ++k) p.c[ax][k] = (A)g.c[ax][k];
-        for (int ax = 0; ax < 3; ++ax)
-            for (int sd = 0; sd < 2; ++sd)
-                for (int k = 0; k < 2; ++k) p.ph[ax][sd][k] = (A)g.phase[ax][sd][k];
-        for (int k = 0; k <= kMaxR; ++k) {
-            q.w1[k] = (A)g.w1[k];
-            q.w2[k] = (A)g.w2[k];
-        }
-        for (int ax = 0; ax < 3; ++ax) q.beta[ax] = (A)g.beta[ax];
-        q.axy_hy = (A)(g.alpha[0] / g.h[1]);
-        q.axz = (A)g.alpha[1];
-        q.ayz = (A)g.alpha[2];
-        q.ihz = (A)(1.0 / g.h[2]);
         for (int i = 0; i < 3; ++i) {
             r.buf[i] = U.buf[i];
             r.ld[i] = U.ld[i];
@@ -2396,46 +1742,27 @@ template <class S, int W, int HP>
 void launch_stencil_batch(const BatchPlan *P, const BatchPlan::SGroup &G, const void *coef, int ix, int iold,
                           int iout, hipStream_t st)
 {
-    using A = typename Tr<S>::A;
     const int blocks = ((G.nitems + 7) / 8) * 8;
-    const auto *recs = static_cast<const BatchRec<A> *>(P->recs);
-    const A *cf = static_cast<const A *>(coef);
+    const auto *recs = static_cast<const BatchRec<S> *>(P->recs);
+    const S *cf = static_cast<const S *>(coef);
     auto go = [&](auto kern, int nt, size_t shm) {
         hipLaunchKernelGGL(kern, dim3(blocks), dim3(nt), shm, st, recs, G.items, G.nitems, cf, ix, iold, iout);
     };
     if constexpr (W == 256) {
-        // long rows: 512 threads, scalar bodies
-        const size_t shm = (G.kind == 1 ? 4 : 2) * sizeof(S) * ((size_t)W * (G.max_tyr + 2 * kMaxR) + 512);
-        if (G.kind == 0) go(k_stencil_batch<S, kMaxR, batch_rp_orth<S>(), 512, kLongHalo, W, 0>, 512, shm);
-        else if constexpr (sizeof(S) <= 8)
-            go(k_stencil_batch<S, kMaxR, batch_rp_nonorth<S>(), 512, kLongHalo, W, 1>, 512, shm);
-    } else if constexpr (W == kShortNonorthPitch) {
-        // short non-orthogonal rows: the tight pitch leaves room for more
-        // workgroups per CU (the body holds four planes of this pitch)
-        const size_t shm = 4 * sizeof(S) * ((size_t)W * (G.max_tyr + 2 * kMaxR) + G.nt);
-        if (G.nt == 192) go(k_stencil_batch<S, kMaxR, batch_rp_nonorth<S>(), 192, 2, W, 1>, 192, shm);
-        else go(k_stencil_batch<S, kMaxR, batch_rp_nonorth<S>(), kBatchNT, HP, W, 1>, kBatchNT, shm);
+        // long rows: 512 threads, scalar body
+        const size_t shm = 2 * sizeof(S) * ((size_t)W * (G.max_tyr + 2 * kMaxR) + 512);
+        go(k_stencil_batch<S, kMaxR, batch_rp_orth<S>(), 512, kLongHalo, W, 0>, 512, shm);
     } else if (G.kind == 2 || G.kind == 3) {
-        if constexpr (!Tr<S>::C) {
-            // vector kinds: halo slots counted in runs (2 or 3 per thread)
-            constexpr int HV = HP == 3 ? 2 : 3;
-            const int VW = G.kind == 3 ? 2 : int(16 / sizeof(S));
-            const size_t shm = 2 * sizeof(S) * ((size_t)W * (G.max_tyr + 2 * kMaxR) + kBatchNT * VW);
-            if (G.kind == 2) go(k_stencil_batch<S, kMaxR, kBatchRuns, kBatchNT, HV, W, 2>, kBatchNT, shm);
-            else if constexpr (sizeof(S) == 4)
-                go(k_stencil_batch<S, kMaxR, kBatchRuns, kBatchNT, HV, W, 3>, kBatchNT, shm);
-        }
-    } else if (G.kind == 1 && G.nt == 192) {
-        // short non-orthogonal rows, two halo slots per thread
-        if constexpr (W == 64) {
-            const size_t shm = 4 * sizeof(S) * ((size_t)W * (G.max_tyr + 2 * kMaxR) + 192);
-            go(k_stencil_batch<S, kMaxR, batch_rp_nonorth<S>(), 192, 2, W, 1>, 192, shm);
-        }
+        // vector kinds: halo slots counted in runs (2 or 3 per thread)
+        constexpr int HV = HP == 3 ? 2 : 3;
+        const int VW = G.kind == 3 ? 2 : int(16 / sizeof(S));
+        const size_t shm = 2 * sizeof(S) * ((size_t)W * (G.max_tyr + 2 * kMaxR) + kBatchNT * VW);
+        if (G.kind == 2) go(k_stencil_batch<S, kMaxR, kBatchRuns, kBatchNT, HV, W, 2>, kBatchNT, shm);
+        else if constexpr (sizeof(S) == 4)
+            go(k_stencil_batch<S, kMaxR, kBatchRuns, kBatchNT, HV, W, 3>, kBatchNT, shm);
     } else {
-        // the non-orthogonal body uses two (plane, g-plane) pairs
-        const size_t shm = (G.kind == 1 ? 4 : 2) * sizeof(S) * ((size_t)W * (G.max_tyr + 2 * kMaxR) + kBatchNT);
-        if (G.kind == 0) go(k_stencil_batch<S, kMaxR, batch_rp_orth<S>(), kBatchNT, HP, W, 0>, kBatchNT, shm);
-        else go(k_stencil_batch<S, kMaxR, batch_rp_nonorth<S>(), kBatchNT, HP, W, 1>, kBatchNT, shm);
+        const size_t shm = 2 * sizeof(S) * ((size_t)W * (G.max_tyr + 2 * kMaxR) + kBatchNT);
+        go(k_stencil_batch<S, kMaxR, batch_rp_orth<S>(), kBatchNT, HP, W, 0>, kBatchNT, shm);
     }
 }
 
@@ -2529,17 +1856,20 @@ void batch_step(BatchPlan *P, int step, int ix, int iold, int iout, hipStream_t 
             else launch_nl_batch<S, 32>(P, G, cf, ix, iout, true, st);
         }
         for (const auto &G : P->sg) {
-            if (G.W == kShortNonorthPitch) {
-                if (G.small_halo) launch_stencil_batch<S, kShortNonorthPitch, 3>(P, G, cf, ix, iold, iout, st);
-                else launch_stencil_batch<S, kShortNonorthPitch, 6>(P, G, cf, ix, iold, iout, st);
-            } else if (G.W == 64) {
-                if (G.small_halo) launch_stencil_batch<S, 64, 3>(P, G, cf, ix, iold, iout, st);
-                else launch_stencil_batch<S, 64, 6>(P, G, cf, ix, iold, iout, st);
-            } else if (G.W == 256) {
-                launch_stencil_batch<S, 256, kLongHalo>(P, G, cf, ix, iold, iout, st);
-            } else {
-                if (G.small_halo) launch_stencil_batch<S, 128, 3>(P, G, cf, ix, iold, iout, st);
-                else launch_stencil_batch<S, 128, 6>(P, G, cf, ix, iold, iout, st);
+            if (G.kind == 1) {
+                points_batch(P->e, P->recs, G.items, G.nitems, G.nonorth, cf, ix, iold, iout, G.shape, st);
+                continue;
+            }
+            if constexpr (!Tr<S>::C) {
+                if (G.W == 64) {
+                    if (G.small_halo) launch_stencil_batch<S, 64, 3>(P, G, cf, ix, iold, iout, st);
+                    else launch_stencil_batch<S, 64, 6>(P, G, cf, ix, iold, iout, st);
+                } else if (G.W == 256) {
+                    launch_stencil_batch<S, 256, kLongHalo>(P, G, cf, ix, iold, iout, st);
+                } else {
+                    if (G.small_halo) launch_stencil_batch<S, 128, 3>(P, G, cf, ix, iold, iout, st);
+                    else launch_stencil_batch<S, 128, 6>(P, G, cf, ix, iold, iout, st);
+                }
             }
         }
         for (const auto &G : P->ng) {

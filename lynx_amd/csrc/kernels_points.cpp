@@ -1,0 +1,89 @@
+// Launch shapes and element-type dispatch of the one-point-per-thread stencil
+// step.
+#include "kernels_points.hpp"
+#include "common.hpp"
+
+#include <algorithm>
+
+namespace lynx {
+namespace gpu {
+
+namespace {
+constexpr long kLds = 160 * 1024;   // LDS of a workgroup (gfx950)
+
+int round64(int n) { return (n + 63) / 64 * 64; }
+}  // namespace
+
+bool point_shape(int e, const StencilGeom &g, int max_threads, int nzch, PointShape &out)
+{
+    const int R = kMaxR, nx = g.nx, ny = g.ny;
+    const long es = (long)elem_size(e);
+    PointShape s;
+    s.pitch = nx + 2 * R <= 40 ? 40 : (nx + 2 * R <= 64 ? 64 : (nx + 2 * R <= 128 ? 128 : 256));
+    // halo points per thread that each pitch's kernels are built for
+    const int slots[4][3] = {{1, 2, 2}, {2, 3, 3}, {2, 3, 6}, {6, 6, 6}};
+    const int *hs = slots[s.pitch == 40 ? 0 : (s.pitch == 64 ? 1 : (s.pitch == 128 ? 2 : 3))];
+    if (nx + 2 * R > 256 || nx > max_threads) return false;
+    s.nzch = std::max(1, std::min(nzch, g.nz));
+    for (int most = std::min(ny, max_threads / nx); most >= 1; --most) {
+        const int nb = (ny + most - 1) / most;
+        s.tyr = (ny + nb - 1) / nb;
+        s.nt = round64(std::max(s.tyr * nx, (2 * R * nx + hs[2] - 1) / hs[2]));
+        if (s.nt > 512) continue;
+        s.hp = hs[2];
+        for (int k = 2; k >= 0; --k)
+            if (2 * R * nx <= hs[k] * s.nt) s.hp = hs[k];
+        const long planes = 2 * es * s.pitch * ((s.tyr + 2 * R) + (g.orth ? 0 : s.tyr));
+        const long stash = 2 * R * es * s.nt;
+        s.wrapz = s.nzch == 1 && g.nz >= 2 * R && planes + stash <= kLds;
+        s.lds = (size_t)(planes + (s.wrapz ? stash : 0));
+        if (planes > kLds) continue;
+        out = s;
+        return true;
+    }
+    return false;
+}
+
+// The cost of a shape per point: idle lanes, halo rows (a tenth of an own
+// row's cost each) and, above 256 threads, fewer workgroups to a CU to hide
+// each other's barriers.  Measured at 24^3 x 1344 complex64: 8 rows in 192
+// threads 176 us, 12 in 320 249 us, 4 in 128 (a quarter of them idle) 218 us,
+// 24 in 576 280 us; at 32^3 x 400: 8 rows in 256 136 us, 4 in 128 160 us,
+// 16 in 512 189 us.
+bool point_shape_batch(int e, const StencilGeom &g, PointShape &out)
+{
+    double best = 0;
+    for (int budget : {128, 192, 256, 320, 384, 448, 512}) {
+        PointShape s;
+        if (!point_shape(e, g, budget, 1, s)) continue;
+        const int nb = (g.ny + s.tyr - 1) / s.tyr;
+        double cost = (double)nb * s.nt / ((double)g.nx * g.ny) * (1.0 + 0.12 * 2 * kMaxR / s.tyr);
+        if (s.nt > 256) cost *= 1.0 + (s.nt - 256) / 400.0;
+        if (best == 0 || cost < best) {
+            best = cost;
+            out = s;
+        }
+    }
+    return best > 0;
+}
+
+void points_step(int e, const StencilGeom &g, const void *x, long ldx, const void *old, long ldo, void *out,
+                 long ldout, const void *veff, int ncol, double a, double b, double s, const PointShape &sh,
+                 hipStream_t st, const void *coef)
+{
+    auto f = e == F64 ? points_step_f64 : e == C128 ? points_step_c128 : e == F32 ? points_step_f32 : points_step_c64;
+    f(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, sh, st, coef);
+}
+
+void points_batch(int e, const void *recs, const int *items, int nitems, bool nonorth, const void *coef, int ix,
+                  int iold, int iout, const PointShape &sh, hipStream_t st)
+{
+    auto f = e == F64   ? points_batch_f64
+             : e == C128 ? points_batch_c128
+             : e == F32  ? points_batch_f32
+                         : points_batch_c64;
+    f(recs, items, nitems, nonorth, coef, ix, iold, iout, sh, st);
+}
+
+}  // namespace gpu
+}  // namespace lynx
