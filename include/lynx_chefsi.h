@@ -569,7 +569,9 @@ lynx_status lynx_batch_set_graph(lynx_batch *batch, int enable);
  * reference filters in FP64). */
 lynx_status lynx_batch_set_filter_precision(lynx_batch *batch, int precision);
 /* Device time of the last lynx_batch_filter (HIP events around the graph
- * launch or the eager launches) and the number of kernel launches it holds. */
+ * launch or the eager launches) and the number of gather, stencil and scatter
+ * kernels it holds (a scatter and the next step's gather in one launch count
+ * as two). */
 lynx_status lynx_batch_last_timing(const lynx_batch *batch, double *ms, int *launches);
 /* One CheFSI pass for every unit of the batch: lynx_chefsi_solve on each
  * unit's block psi[u] (device memory, leading dimension ldpsi[u], ncol[u]

@@ -29,6 +29,7 @@ SOURCES = [
     ("kernels_scf.hip", "hip"),
     ("kernels_mfma.hip", "hip"),
     ("kernels_dense.hip", "hip"),
+    ("kernels_nonlocal.hip", "hip"),
     ("kernels_points.cpp", "hip"),
     ("kernels_points_f64.hip", "hip"),
     ("kernels_points_c128.hip", "hip"),

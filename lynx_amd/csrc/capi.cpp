@@ -5,6 +5,7 @@
 #include "lynx_chefsi.h"
 
 #include "ctx.hpp"
+#include "kernels_nonlocal.hpp"
 
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
@@ -254,6 +255,7 @@ void upload_nonlocal(lynx_ctx *c)
         v->n_cov = (int)cov_gpos.size();
         v->n_img = h.n_img;
         v->max_atom_pts = 0;
+        v->disjoint = npts == (int)cov_gpos.size();
         for (int a = 0; a < h.n_atom; ++a)
             v->max_atom_pts = std::max(v->max_atom_pts, atom_pt_off[a + 1] - atom_pt_off[a]);
         v->atom_pt_off = c->d_atom_pt_off.as<int>();
@@ -390,26 +392,40 @@ bool bf16_filter_fits(const lynx_ctx *c)
 }
 
 // ------------------------------------------------------------- operator --
+// The two tables of projector coefficients of a filter's steps (taken in
+// turn: an update reads one and writes the other); applies use the first.
+void *beta_table(lynx_ctx *c, int e, int ncol, int which)
+{
+    const gpu::NlDev &nd = nl_for(c, e);
+    const size_t bytes = ((size_t)ncol * nd.n_atom * nd.npm * gpu::elem_size(gpu::elem_compute(e)) + 255) / 256 * 256;
+    return static_cast<char *>(c->beta.get(2 * bytes)) + which * bytes;
+}
+
+void local_step(lynx_ctx *c, int e, const void *x, long ldx, const void *old, long ldo, void *y, long ldy, int ncol,
+                double a, double b, double shift, const void *coef)
+{
+    const gpu::StepCfg cfg = step_config(c, e, x, ldx, y, ldy, ncol);
+    Marker m(c, 1);
+    gpu::stencil_step(e, geom(c), x, ldx, old, ldo, y, ldy, veff_for(c, e), ncol, a, b, shift, cfg, c->stream, coef);
+}
+
 // y = a * (H - shift) x + b * old, H = -1/2 lap + Veff + V_nl.
 void apply_op(lynx_ctx *c, int e, const void *x, long ldx, const void *old, long ldo, void *y, long ldy,
               int ncol, double a, double b, double shift, const void *coef = nullptr)
 {
-    const gpu::StepCfg cfg = step_config(c, e, x, ldx, y, ldy, ncol);
     const bool nl = c->has_nl;
     const gpu::NlDev &nd = nl_for(c, e);
+    // the launch shape is tuned before the gather (the tuner writes y)
+    (void)step_config(c, e, x, ldx, y, ldy, ncol);
     if (nl) {
-        c->beta.get((size_t)ncol * nd.n_atom * nd.npm * gpu::elem_size(gpu::elem_compute(e)));
+        void *beta = beta_table(c, e, ncol, 0);
         Marker m(c, 2);
-        gpu::nl_gather(e, nd, x, ldx, c->beta.p, ncol, c->stream);
+        gpu::nl_gather(e, nd, x, ldx, beta, ncol, c->stream);
     }
-    {
-        Marker m(c, 1);
-        gpu::stencil_step(e, geom(c), x, ldx, old, ldo, y, ldy, veff_for(c, e), ncol, a, b, shift, cfg,
-                          c->stream, coef);
-    }
+    local_step(c, e, x, ldx, old, ldo, y, ldy, ncol, a, b, shift, coef);
     if (nl) {
         Marker m(c, 3);
-        gpu::nl_scatter(e, nd, c->beta.p, y, ldy, ncol, a, c->stream, coef);
+        gpu::nl_scatter(e, nd, beta_table(c, e, ncol, 0), y, ldy, ncol, a, c->stream, coef);
     }
     HIP_OK(hipGetLastError());
 }
@@ -457,19 +473,38 @@ void filter(lynx_ctx *c, int e, const void *x, long ldx, void *y, long ldy, void
         auto cf = [&](int k) -> const void * {
             return table ? static_cast<const char *>(c->fcoef.p) + (size_t)3 * (k - 1) * ce : nullptr;
         };
-        apply_op(c, e, x, ldx, nullptr, 0, D1, ld1, ncol, sc[0], sc[1], sc[2], cf(1));
-        const void *prev = D1;   // Y_{k-1}
-        long ldp = ld1;
-        const void *pprev = x;   // Y_{k-2}
-        long ldpp = ldx;
-        for (int k = 2; k <= degree; ++k) {
+        const gpu::NlDev &nd = nl_for(c, e);
+        // spheres without common grid points: the scatter of a step and the
+        // gather of the next one, which reads the same points of the block
+        // it has completed, are one pass
+        const bool fused = c->has_nl && gpu::nl_tile_fits(nd, gpu::kNlUpdate);
+        const void *prev = x, *pprev = nullptr;   // Y_{k-1}, Y_{k-2}
+        long ldp = ldx, ldpp = 0;
+        for (int k = 1; k <= degree; ++k) {
             void *dst = (k % 2 == 1) ? D1 : D2;
             const long ldd = (k % 2 == 1) ? ld1 : ld2;
-            apply_op(c, e, prev, ldp, pprev, ldpp, dst, ldd, ncol, sc[3 * (k - 1)], sc[3 * (k - 1) + 1],
-                     sc[3 * (k - 1) + 2], cf(k));
+            const double *q = &sc[3 * (k - 1)];
+            if (!fused) {
+                apply_op(c, e, prev, ldp, pprev, ldpp, dst, ldd, ncol, q[0], q[1], q[2], cf(k));
+            } else {
+                if (k == 1) {
+                    (void)step_config(c, e, prev, ldp, dst, ldd, ncol);
+                    Marker m(c, 2);
+                    gpu::nl_gather(e, nd, prev, ldp, beta_table(c, e, ncol, 0), ncol, c->stream);
+                }
+                local_step(c, e, prev, ldp, pprev, ldpp, dst, ldd, ncol, q[0], q[1], q[2], cf(k));
+                Marker m(c, 3);
+                void *bt = beta_table(c, e, ncol, (k - 1) & 1);
+                if (k < degree)
+                    gpu::nl_tile(e, nd, gpu::kNlUpdate, bt, beta_table(c, e, ncol, k & 1), dst, ldd, ncol, q[0],
+                                 c->stream, cf(k));
+                else
+                    gpu::nl_scatter(e, nd, bt, dst, ldd, ncol, q[0], c->stream, cf(k));
+            }
             pprev = prev; ldpp = ldp;
             prev = dst; ldp = ldd;
         }
+        HIP_OK(hipGetLastError());
     };
     if (!c->use_graphs || degree > kMaxGraphDegree) {
         run(false);
@@ -478,8 +513,7 @@ void filter(lynx_ctx *c, int e, const void *x, long ldx, void *y, long ldy, void
     const gpu::StepCfg cfg = step_config(c, e, x, ldx, D1, ld1, ncol);
     if (c->has_nl) {
         // beta sized before the key: the graph's launches hold its address
-        const gpu::NlDev &nd = nl_for(c, e);
-        c->beta.get((size_t)ncol * nd.n_atom * nd.npm * gpu::elem_size(gpu::elem_compute(e)));
+        (void)beta_table(c, e, ncol, 0);
     }
     // everything a captured launch holds by value: buffers, shapes, the
     // set-up epoch (grid, atoms, projectors, forced launch shapes), Veff and
@@ -2220,12 +2254,12 @@ lynx_status lynx_batch_filter(lynx_batch *b, int dtype, void *const *x, const lo
         }
         gpu::batch_set_coef(b->plan, coef.data(), degree, b->stream);
         auto record = [&] {
-            gpu::batch_step(b->plan, 0, 0, 3, 1, b->stream);
+            gpu::batch_step(b->plan, 0, 0, 3, 1, true, degree == 1, b->stream);
             int prev = 1;
             for (int k = 2; k <= degree; ++k) {
                 const int dst = (k % 2 == 1) ? 1 : 2;
                 const int old = (k == 2) ? 0 : dst;
-                gpu::batch_step(b->plan, k - 1, prev, old, dst, b->stream);
+                gpu::batch_step(b->plan, k - 1, prev, old, dst, false, k == degree, b->stream);
                 prev = dst;
             }
         };
@@ -2261,7 +2295,7 @@ lynx_status lynx_batch_filter(lynx_batch *b, int dtype, void *const *x, const lo
         float ms = 0;
         HIP_OK(hipEventElapsedTime(&ms, b->e0, b->e1));
         b->last_ms = ms;
-        b->last_launches = degree * gpu::batch_launches_per_step(b->plan);
+        b->last_launches = gpu::batch_launches(b->plan, degree);
     });
 }
 
@@ -2501,7 +2535,7 @@ lynx_status lynx_batch_solve(lynx_batch *b, int dtype, void *const *psi, const l
             std::vector<double> coef((size_t)n * 3, 0.0);
             for (int u = 0; u < n; ++u) coef[3 * u] = 1.0;
             gpu::batch_set_coef(b->hplan, coef.data(), 1, st);
-            gpu::batch_step(b->hplan, 0, 0, 3, 1, st);
+            gpu::batch_step(b->hplan, 0, 0, 3, 1, true, true, st);
         }
         // 4. Rayleigh-Ritz per group: Hs = dV psi^H (H psi), Hermitian part,
         // Hs = Q Lambda Q^H, psi = psi Q (EigenSolver.cpp:643-681)

@@ -3,6 +3,7 @@
 // small helpers.  Launch wrappers at the bottom.
 #include "kernels.hpp"
 #include "common.hpp"
+#include "kernels_nonlocal.hpp"
 #include "kernels_points.hpp"
 #include "stencil_common.hpp"
 
@@ -633,30 +634,27 @@ __global__ void __launch_bounds__(NT) k_stencil_vacc(StepArgs<S> p)
 }
 
 // --------------------------------------------------------- nonlocal gather --
-// One workgroup per (physical atom, column).  The four waves take
-// interleaved runs of the atom's sphere points (all images); each lane
-// accumulates npm projections, then a wave reduction, and the four wave sums
-// are added in a fixed order through LDS (deterministic, no atomics).
-// SPLIT = false: one wave per column (four columns per workgroup, index c
-// is the column group); SPLIT = true: the four waves share one column (c)
-// and split the points, for atoms with many sphere points.
-template <class S, int NPM, bool SPLIT, class T = S>
-__device__ __forceinline__ void nl_gather_body(const NlArgs<typename Tr<S>::A> &p, const T *__restrict__ X,
-                                               long ldx, S *__restrict__ beta, int ncol, int at, int c)
+// Atoms of more than kTileAtomPts sphere points (smaller ones:
+// kernels_nonlocal.hip): one workgroup per (physical atom, column).  The four
+// waves take interleaved runs of the atom's sphere points (all images); each
+// lane accumulates npm projections, then a wave reduction, and the four wave
+// sums are added in a fixed order through LDS (deterministic, no atomics).
+template <class S, int NPM, class T>
+__global__ void __launch_bounds__(256) k_nl_gather(NlArgs<typename Tr<S>::A> p, const T *__restrict__ X,
+                                                   long ldx, S *__restrict__ beta, int ncol)
 {
     using A = typename Tr<S>::A;
     __shared__ S part[4][NPM];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    const int n = SPLIT ? c : c * 4 + wave;
-    if (n >= ncol) return;       // uniform over the workgroup when SPLIT
+    const int at = blockIdx.x, n = blockIdx.y;
+    if (n >= ncol) return;
     const int pb = p.atom_pt_off[at], pe = p.atom_pt_off[at + 1];
     const T *Xn = X + (long)n * ldx;
     S acc[NPM];
 #pragma unroll
     for (int j = 0; j < NPM; ++j) acc[j] = zero<S>();
-    constexpr int kStride = SPLIT ? 256 : 64;
-    for (int e = pb + (SPLIT ? wave * 64 : 0) + lane; e < pe; e += kStride) {
+    for (int e = pb + wave * 64 + lane; e < pe; e += 256) {
         S v = to_compute(Xn[p.pt_gpos[e]]);
         if constexpr (Tr<S>::C) {
             const int im = p.pt_img[e];
@@ -678,13 +676,6 @@ __device__ __forceinline__ void nl_gather_body(const NlArgs<typename Tr<S>::A> &
             }
         }
     }
-    if constexpr (!SPLIT) {
-        S *bn = beta + (long)n * p.n_atom * NPM + (long)at * NPM;
-#pragma unroll
-        for (int j = 0; j < NPM; ++j)
-            if (lane == j) bn[j] = scl(p.gamma[at * NPM + j], acc[j]);
-        return;
-    }
 #pragma unroll
     for (int j = 0; j < NPM; ++j)
         if (lane == j) part[wave][j] = acc[j];
@@ -698,17 +689,6 @@ __device__ __forceinline__ void nl_gather_body(const NlArgs<typename Tr<S>::A> &
         bn[lane] = scl(p.gamma[at * NPM + lane], t);
     }
 }
-
-template <class S, int NPM, bool SPLIT, class T>
-__global__ void __launch_bounds__(256) k_nl_gather(NlArgs<typename Tr<S>::A> p, const T *__restrict__ X,
-                                                   long ldx, S *__restrict__ beta, int ncol)
-{
-    nl_gather_body<S, NPM, SPLIT, T>(p, X, ldx, beta, ncol, blockIdx.x, blockIdx.y);
-}
-
-// atoms with more sphere points than this are gathered by four waves (one
-// operator) or by parts (batches, k_nl_gather_part_batch)
-constexpr int kGatherSplitPts = 1024;
 
 // -------------------------------------------------------- nonlocal scatter --
 // Owner-computes: one lane per covered grid point, one wave per column; sums
@@ -830,24 +810,6 @@ __global__ void __launch_bounds__(NT) k_stencil_batch(const BatchRec<S> *__restr
         stencil_vacc_body<S, R, RP, NT, HP, W, 2, KIND == 3 ? 2 : int(16 / sizeof(S))>(r.q.b, io, w - r.item0);
     else
         stencil_step_body<S, R, RP, NT, HP, W>(r.q.b, io, w - r.item0);
-}
-
-// Batched gather of units whose atoms have small spheres: one workgroup per
-// (atom, group of four columns), one wave per column.
-template <class S, int NPM>
-__global__ void __launch_bounds__(256) k_nl_gather_batch(const BatchRec<typename Tr<S>::A> *__restrict__ recs,
-                                                         const int *__restrict__ item_unit, int nitems,
-                                                         S *__restrict__ beta, int ix)
-{
-    using A = typename Tr<S>::A;
-    const int w = blockIdx.x;
-    if (w >= nitems) return;
-    const int u = item_unit[w];
-    const BatchRec<A> &r = recs[u];
-    const NlArgs<A> nl = r.nl;
-    const int lb = w - r.g_item0;
-    nl_gather_body<S, NPM, false>(nl, reinterpret_cast<const S *>(r.buf[ix]), r.ld[ix], beta + r.beta_off,
-                                  r.ncol, lb % nl.n_atom, lb / nl.n_atom);
 }
 
 // Gather by parts, for units whose atoms have large spheres: one workgroup
@@ -1416,15 +1378,8 @@ static void gather_npm(const NlDev &nl, const void *x, long ldx, void *beta, int
     using A = typename Tr<S>::A;
     NlArgs<A> p{nl.atom_pt_off, nl.pt_gpos, nl.pt_img, nl.pt_atom, nl.cov_off, nl.cov_gpos, nl.ent_pt,
                 (const A *)nl.chi, (const A *)nl.gamma, (const A *)nl.phase, nl.n_atom, nl.n_cov, nl.npm};
-    if (nl.max_atom_pts > kGatherSplitPts) {
-        dim3 grid(nl.n_atom, ncol);
-        hipLaunchKernelGGL((k_nl_gather<S, NPM, true, T>), grid, dim3(256), 0, st, p, (const T *)x, ldx,
-                           (S *)beta, ncol);
-    } else {
-        dim3 grid(nl.n_atom, (ncol + 3) / 4);
-        hipLaunchKernelGGL((k_nl_gather<S, NPM, false, T>), grid, dim3(256), 0, st, p, (const T *)x, ldx,
-                           (S *)beta, ncol);
-    }
+    hipLaunchKernelGGL((k_nl_gather<S, NPM, T>), dim3(nl.n_atom, ncol), dim3(256), 0, st, p, (const T *)x, ldx,
+                       (S *)beta, ncol);
 }
 
 template <class S, int NPM, class T = S>
@@ -1443,6 +1398,10 @@ static void scatter_npm(const NlDev &nl, const void *beta, void *y, long ldy, in
 void nl_gather(int e, const NlDev &nl, const void *x, long ldx, void *beta, int ncol, hipStream_t st)
 {
     if (nl.n_atom == 0 || nl.n_pts == 0) return;
+    if (nl_tile_fits(nl, kNlGather)) {
+        nl_tile(e, nl, kNlGather, nullptr, beta, const_cast<void *>(x), ldx, ncol, 0.0, st);
+        return;
+    }
     if (e == B16) {
         // bfloat16 storage: x read as bf16, beta in float
         if (nl.npm == 8) gather_npm<float, 8, bf16>(nl, x, ldx, beta, ncol, st);
@@ -1494,12 +1453,15 @@ struct BatchPlan {
     struct NGroup {
         int npm = 8;
         bool split = false;     // gather by parts (k_nl_gather_part_batch), then a reduction
+        bool update = false;    // no grid point in two spheres: scatter and next gather in one launch
+        int waves = 1;          // of a gather / update workgroup (not split)
         int *gitems = nullptr, *sitems = nullptr, *ritems = nullptr;
         int ngitems = 0, nsitems = 0, nritems = 0;
     };
     std::vector<SGroup> sg;
     std::vector<NGroup> ng;
     void *beta = nullptr;
+    size_t beta_bytes = 0;
     void *partial = nullptr;    // part sums of the gather by parts
     int2 *parts = nullptr;      // part point ranges, all units
     int *atom_part = nullptr;   // first part of each atom, all units
@@ -1592,18 +1554,21 @@ void build_batch(BatchPlan *P, const BatchUnit *units, int n, hipStream_t st)
         sgi[u] = k;
         P->sg[k].shape.lds = std::max(P->sg[k].shape.lds, shape[u].lds);
         if (units[u].nl.n_atom > 0 && units[u].nl.n_pts > 0) {
-            const bool split = units[u].nl.max_atom_pts > kGatherSplitPts;
+            const bool split = !nl_tile_fits(units[u].nl, kNlGather);
+            const bool update = nl_tile_fits(units[u].nl, kNlUpdate);
             int j = -1;
             for (size_t i = 0; i < P->ng.size(); ++i)
-                if (P->ng[i].npm == units[u].nl.npm && P->ng[i].split == split) j = (int)i;
+                if (P->ng[i].npm == units[u].nl.npm && P->ng[i].split == split && P->ng[i].update == update) j = (int)i;
             if (j < 0) {
                 BatchPlan::NGroup G;
                 G.npm = units[u].nl.npm;
                 G.split = split;
+                G.update = update;
                 P->ng.push_back(G);
                 j = (int)P->ng.size() - 1;
             }
             ngi[u] = j;
+            P->ng[j].waves = std::max(P->ng[j].waves, nl_tile_waves(units[u].nl.max_atom_pts));
         }
     }
     std::vector<std::vector<int>> sitems(P->sg.size()), gitems(P->ng.size()), citems(P->ng.size()),
@@ -1697,8 +1662,7 @@ void build_batch(BatchPlan *P, const BatchUnit *units, int n, hipStream_t st)
                 const long nred = (long)U.ncol * nl.n_atom * nl.npm;
                 for (long w = 0; w < (nred + 255) / 256; ++w) ri.push_back(u);
             } else {
-                // (atom, group of four columns)
-                const int cg = (U.ncol + 3) / 4;
+                const int cg = nl_tile_groups(P->e, U.ncol);
                 for (int w = 0; w < nl.n_atom * cg; ++w) gi.push_back(u);
             }
             // scatter: column groups of 4 cpw columns, cpw chosen so the
@@ -1734,7 +1698,9 @@ void build_batch(BatchPlan *P, const BatchUnit *units, int n, hipStream_t st)
         P->ng[i].nritems = (int)ritems[i].size();
         P->ng[i].ritems = dev_upload(ritems[i], st);
     }
-    hip_check(hipMalloc(&P->beta, std::max<size_t>(1, beta_off * sizeof(S))), "hipMalloc");
+    // two tables in turn: an update reads one and writes the other
+    P->beta_bytes = (beta_off * sizeof(S) + 255) / 256 * 256;
+    hip_check(hipMalloc(&P->beta, std::max<size_t>(1, 2 * P->beta_bytes)), "hipMalloc");
     hip_check(hipStreamSynchronize(st), "batch upload");
 }
 
@@ -1767,27 +1733,32 @@ void launch_stencil_batch(const BatchPlan *P, const BatchPlan::SGroup &G, const 
 }
 
 template <class S, int NPM>
-void launch_nl_batch(const BatchPlan *P, const BatchPlan::NGroup &G, const void *coef, int ix, int iout,
-                     bool gather, hipStream_t st)
+void launch_nl_split_batch(const BatchPlan *P, const BatchPlan::NGroup &G, int ix, hipStream_t st)
 {
     using A = typename Tr<S>::A;
     const auto *recs = static_cast<const BatchRec<A> *>(P->recs);
-    if (gather) {
-        if (G.ngitems > 0) {
-            if (G.split) {
-                hipLaunchKernelGGL((k_nl_gather_part_batch<S, NPM>), dim3(G.ngitems), dim3(256), 0, st, recs,
-                                   G.gitems, G.ngitems, static_cast<S *>(P->partial), ix);
-                hipLaunchKernelGGL((k_nl_gather_reduce_batch<S, NPM>), dim3(G.nritems), dim3(256), 0, st, recs,
-                                   G.ritems, G.nritems, static_cast<const S *>(P->partial),
-                                   static_cast<S *>(P->beta));
-            } else
-                hipLaunchKernelGGL((k_nl_gather_batch<S, NPM>), dim3(G.ngitems), dim3(256), 0, st, recs,
-                                   G.gitems, G.ngitems, static_cast<S *>(P->beta), ix);
-        }
-    } else if (G.nsitems > 0) {
-        hipLaunchKernelGGL((k_nl_scatter_batch<S, NPM>), dim3(G.nsitems), dim3(256), 0, st, recs, G.sitems,
-                           G.nsitems, static_cast<const S *>(P->beta), static_cast<const A *>(coef), iout);
-    }
+    hipLaunchKernelGGL((k_nl_gather_part_batch<S, NPM>), dim3(G.ngitems), dim3(256), 0, st, recs, G.gitems, G.ngitems,
+                       static_cast<S *>(P->partial), ix);
+    hipLaunchKernelGGL((k_nl_gather_reduce_batch<S, NPM>), dim3(G.nritems), dim3(256), 0, st, recs, G.ritems,
+                       G.nritems, static_cast<const S *>(P->partial), static_cast<S *>(P->beta));
+}
+
+template <class S, int NPM>
+void launch_nl_scatter_batch(const BatchPlan *P, const BatchPlan::NGroup &G, const void *beta, const void *coef,
+                             int iout, hipStream_t st)
+{
+    using A = typename Tr<S>::A;
+    hipLaunchKernelGGL((k_nl_scatter_batch<S, NPM>), dim3(G.nsitems), dim3(256), 0, st,
+                       static_cast<const BatchRec<A> *>(P->recs), G.sitems, G.nsitems,
+                       static_cast<const S *>(beta), static_cast<const A *>(coef), iout);
+}
+
+template <class F>
+void by_npm(int npm, F &&f)
+{
+    if (npm == 8) f(std::integral_constant<int, 8>{});
+    else if (npm == 16) f(std::integral_constant<int, 16>{});
+    else f(std::integral_constant<int, 32>{});
 }
 }  // namespace
 
@@ -1843,17 +1814,23 @@ void batch_set_coef(BatchPlan *P, const double *coef, int steps, hipStream_t st)
     }
 }
 
-void batch_step(BatchPlan *P, int step, int ix, int iold, int iout, hipStream_t st)
+void batch_step(BatchPlan *P, int step, int ix, int iold, int iout, bool first, bool last, hipStream_t st)
 {
     if (step >= P->coef_steps) fail(1, "batch step beyond the uploaded filter coefficients");
+    char *beta[2] = {static_cast<char *>(P->beta), static_cast<char *>(P->beta) + P->beta_bytes};
     dispatch(P->e, [&](auto t) {
         using S = decltype(t);
         using A = typename Tr<S>::A;
         const void *cf = static_cast<const A *>(P->coef) + (size_t)step * P->n * 3;
+        // update groups: beta[step % 2] holds this step's coefficients, from
+        // the first gather or the step before
         for (const auto &G : P->ng) {
-            if (G.npm == 8) launch_nl_batch<S, 8>(P, G, cf, ix, iout, true, st);
-            else if (G.npm == 16) launch_nl_batch<S, 16>(P, G, cf, ix, iout, true, st);
-            else launch_nl_batch<S, 32>(P, G, cf, ix, iout, true, st);
+            if (G.ngitems == 0 || (G.update && !first)) continue;
+            if (G.split)
+                by_npm(G.npm, [&](auto np) { launch_nl_split_batch<S, decltype(np)::value>(P, G, ix, st); });
+            else
+                nl_tile_batch(P->e, G.npm, P->recs, G.gitems, G.ngitems, G.waves, kNlGather, nullptr,
+                              G.update ? beta[step & 1] : beta[0], cf, ix, st);
         }
         for (const auto &G : P->sg) {
             if (G.kind == 1) {
@@ -1873,18 +1850,22 @@ void batch_step(BatchPlan *P, int step, int ix, int iold, int iout, hipStream_t 
             }
         }
         for (const auto &G : P->ng) {
-            if (G.npm == 8) launch_nl_batch<S, 8>(P, G, cf, ix, iout, false, st);
-            else if (G.npm == 16) launch_nl_batch<S, 16>(P, G, cf, ix, iout, false, st);
-            else launch_nl_batch<S, 32>(P, G, cf, ix, iout, false, st);
+            const void *bt = G.update ? beta[step & 1] : beta[0];
+            if (G.update && !last)
+                nl_tile_batch(P->e, G.npm, P->recs, G.gitems, G.ngitems, G.waves, kNlUpdate, bt, beta[(step & 1) ^ 1],
+                              cf, iout, st);
+            else if (G.nsitems > 0)
+                by_npm(G.npm,
+                       [&](auto np) { launch_nl_scatter_batch<S, decltype(np)::value>(P, G, bt, cf, iout, st); });
         }
     });
 }
 
-int batch_launches_per_step(const BatchPlan *P)
+int batch_launches(const BatchPlan *P, int steps)
 {
     int n = (int)(P->sg.size() + 2 * P->ng.size());
     for (const auto &G : P->ng) n += G.split && G.ngitems > 0;   // the part sums' reduction
-    return n;
+    return n * steps;
 }
 
 void gram_reduce(int e, const void *work, int nsplit, int n, double alpha, void *C, hipStream_t st)

@@ -61,6 +61,7 @@ bool stencil_shape_fits(int e, int nx, const StepCfg &cfg);
 struct NlDev {
     int n_atom = 0, npm = 0, n_pts = 0, n_cov = 0, n_img = 0;
     int max_atom_pts = 0;               // most sphere points of one atom (all images)
+    bool disjoint = false;              // no grid point lies in two spheres
     const int *atom_pt_off = nullptr;   // n_atom+1
     const int *pt_gpos = nullptr;       // n_pts
     const int *pt_img = nullptr;        // n_pts
@@ -101,9 +102,15 @@ void batch_plan_destroy(BatchPlan *p);
 // Filter scalars of every step: coef[(step * n + u) * 3 + {0, 1, 2}] = (a, b, s).
 void batch_set_coef(BatchPlan *p, const double *coef, int steps, hipStream_t st);
 // One recurrence step for every unit: buf[iout] = a (H - shift) buf[ix] + b buf[iold]
-// (iold = 3: no old term).  Launches gather, stencil and scatter per group.
-void batch_step(BatchPlan *p, int step, int ix, int iold, int iout, hipStream_t st);
-int batch_launches_per_step(const BatchPlan *p);
+// (iold = 3: no old term): the gather, the stencil and the scatter per group.
+// Where a unit's spheres share no grid point, the scatter of a step and the
+// gather of the next one (whose input it has just completed) are one launch:
+// first and last mark the ends of a run of steps, each step taking the output
+// of the one before.
+void batch_step(BatchPlan *P, int step, int ix, int iold, int iout, bool first, bool last, hipStream_t st);
+// Gather, stencil and scatter kernels of a run of steps; a scatter and gather
+// in one launch count as two.
+int batch_launches(const BatchPlan *P, int steps);
 
 // C (n x n) = alpha * sum of nsplit consecutive n x n partial products in work
 // (fixed order).  C is FP64 (F64 or C128) whatever the precision e of the
