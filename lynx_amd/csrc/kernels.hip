@@ -38,6 +38,9 @@ struct StepLoads {
     S halo[HP];                  // halo-row values of plane z
 };
 
+// halo slots per thread of the scalar body (rows of up to 256 points)
+constexpr int kLongHalo = 6;
+
 template <class S, int R, int RP, int NT, int HP, int W>
 __device__ __forceinline__ void stencil_step_body(const StepArgs<typename Tr<S>::A> &p, const StepIO<typename Tr<S>::A> io, const int w)
 {
@@ -65,9 +68,9 @@ __device__ __forceinline__ void stencil_step_body(const StepArgs<typename Tr<S>:
     const int z1 = min(z0 + p.zch, nz);
     const int nxny = nx * ny;
 
-    const S *__restrict__ X = reinterpret_cast<const S *>(io.x) + (long)col * io.ldx;
-    const S *__restrict__ O = reinterpret_cast<const S *>(io.old) + (long)col * io.ldo;
-    S *__restrict__ Y = reinterpret_cast<S *>(io.out) + (long)col * io.ldout;
+    const S *__restrict__ X = global_ptr(reinterpret_cast<const S *>(io.x)) + (long)col * io.ldx;
+    const S *__restrict__ O = global_ptr(reinterpret_cast<const S *>(io.old)) + (long)col * io.ldo;
+    S *__restrict__ Y = global_ptr(reinterpret_cast<S *>(io.out)) + (long)col * io.ldout;
     const bool has_old = io.old != nullptr && io.b != A(0);   // no Y_(k-2) stream without a buffer
 
     const int tid = threadIdx.x;
@@ -126,7 +129,7 @@ __device__ __forceinline__ void stencil_step_body(const StepArgs<typename Tr<S>:
         load_plane(zs + R, L.front);
         const int zo = zs * nxny;
         const S *Oz = O + zo;
-        const A *Vz = p.veff + zo;
+        const A *Vz = global_ptr(p.veff) + zo;
         const S *Xz = X + zo;
 #pragma unroll
         for (int r = 0; r < RP; ++r) {
@@ -791,14 +794,12 @@ __global__ void __launch_bounds__(256) k_nl_scatter_mc(NlArgs<typename Tr<S>::A>
 // kernel covers every unit.  Work items of a unit are contiguous, so the
 // XCD-aware order keeps a unit's bands on one XCD; a table maps each work
 // item to its unit.
-// KIND: 0 real orthogonal units, scalar body; 2 the same with 16-byte runs
-// and row-aligned lanes (RP runs per thread; the forward-accumulation body
-// with loads two planes ahead); 3 the same with 8-byte runs of two floats.
-// Complex and non-orthogonal units (kind 1) run in points_batch.
-template <class S, int R, int RP, int NT, int HP, int W, int KIND>
-__global__ void __launch_bounds__(NT) k_stencil_batch(const BatchRec<S> *__restrict__ recs,
-                                                      const int *__restrict__ item_unit, int nitems,
-                                                      const S *__restrict__ coef, int ix, int iold, int iout)
+// Real orthogonal units with rows of more than 116 points; all others run in
+// points_batch.
+template <class S, int RP>
+__global__ void __launch_bounds__(512) k_stencil_batch(const BatchRec<S> *__restrict__ recs,
+                                                       const int *__restrict__ item_unit, int nitems,
+                                                       const S *__restrict__ coef, int ix, int iold, int iout)
 {
     const int w = xcd_work_item();
     if (w >= nitems) return;
@@ -806,10 +807,7 @@ __global__ void __launch_bounds__(NT) k_stencil_batch(const BatchRec<S> *__restr
     const BatchRec<S> &r = recs[u];
     const StepIO<S> io{r.buf[ix], r.buf[iold], const_cast<void *>(r.buf[iout]), r.ld[ix], r.ld[iold], r.ld[iout],
                        coef[3 * u], coef[3 * u + 1], coef[3 * u + 2]};
-    if constexpr (KIND == 2 || KIND == 3)
-        stencil_vacc_body<S, R, RP, NT, HP, W, 2, KIND == 3 ? 2 : int(16 / sizeof(S))>(r.q.b, io, w - r.item0);
-    else
-        stencil_step_body<S, R, RP, NT, HP, W>(r.q.b, io, w - r.item0);
+    stencil_step_body<S, kMaxR, RP, 512, kLongHalo, 256>(r.q.b, io, w - r.item0);
 }
 
 // Gather by parts, for units whose atoms have large spheres: one workgroup
@@ -837,14 +835,14 @@ __global__ void __launch_bounds__(256) k_nl_gather_part_batch(const BatchRec<typ
     if (w >= nitems) return;
     const int u = item_unit[w];
     const BatchRec<A> &r = recs[u];
-    const NlArgs<A> nl = r.nl;
+    const NlArgs<A> nl = global_args(r.nl);
     const int lb = w - r.g_item0;
     const int q = lb % r.nparts;
     const int c0 = (lb / r.nparts) * CG;
     const int ncol = r.ncol;
-    const int2 pr = r.parts[q];
+    const int2 pr = global_ptr(r.parts)[q];
     const int np = pr.y - pr.x;
-    const S *__restrict__ X = reinterpret_cast<const S *>(r.buf[ix]);
+    const S *__restrict__ X = global_ptr(reinterpret_cast<const S *>(r.buf[ix]));
     const long ldx = r.ld[ix];
     const int tid = threadIdx.x;
     for (int i = tid; i < CG * PP; i += 256) {
@@ -894,14 +892,15 @@ __global__ void __launch_bounds__(256) k_nl_gather_reduce_batch(const BatchRec<t
     if (w >= nitems) return;
     const int u = item_unit[w];
     const BatchRec<A> &r = recs[u];
-    const NlArgs<A> nl = r.nl;
+    const NlArgs<A> nl = global_args(r.nl);
     const long i = (long)(w - r.r_item0) * 256 + threadIdx.x;
     if (i >= (long)r.ncol * nl.n_atom * NPM) return;
     const int jj = (int)(i % NPM);
     const int at = (int)((i / NPM) % nl.n_atom);
     const int c = (int)(i / ((long)NPM * nl.n_atom));
     S t = zero<S>();
-    const int q0 = r.atom_part[at], q1 = r.atom_part[at + 1];
+    const int *ap = global_ptr(r.atom_part);
+    const int q0 = ap[at], q1 = ap[at + 1];
     // loads issued four parts ahead; the sum stays in part order
 #pragma unroll 4
     for (int q = q0; q < q1; ++q) t = add(t, partial[r.part_off + ((long)q * r.ncol + c) * NPM + jj]);
@@ -922,11 +921,11 @@ __global__ void __launch_bounds__(256) k_nl_scatter_batch(const BatchRec<typenam
     if (w >= nitems) return;
     const int u = item_unit[w];
     const BatchRec<A> &r = recs[u];
-    const NlArgs<A> nl = r.nl;
+    const NlArgs<A> nl = global_args(r.nl);
     const int lb = w - r.s_item0;
     const int ncb = (nl.n_cov + 63) / 64;
     nl_scatter_mc_body<S, NPM, kBatchScatterCpw, S>(nl, beta + r.beta_off,
-                                                    reinterpret_cast<S *>(const_cast<void *>(r.buf[iout])),
+                                                    global_ptr(reinterpret_cast<S *>(const_cast<void *>(r.buf[iout]))),
                                                     r.ld[iout], r.ncol, coef[3 * u], lb % ncb, lb / ncb, r.s_cpw);
 }
 
@@ -1111,7 +1110,6 @@ int nonorth_max_rows(int pitch, int nt)
 // points: 64, 128, or 256 for long rows (nx + 2R > 128; 512-thread shapes,
 // with kLongHalo halo slots per thread for up to 256-point rows)
 inline int tile_pitch(int nx) { return nx + 2 * kMaxR <= 64 ? 64 : (nx + 2 * kMaxR <= 128 ? 128 : 256); }
-constexpr int kLongHalo = 6;
 
 // rows per band of the scalar body within the LDS: two planes of
 // pitch * (rows + 2R) + NT elements
@@ -1139,8 +1137,6 @@ void launch_step_rp(const StencilGeom &g, const void *x, long ldx, const void *o
                     int nzch, hipStream_t st, const void *coef = nullptr)
 {
     using A = typename Tr<S>::A;
-    constexpr int HS = NT >= 512 ? 2 : 3;      // halo slots: rows up to 64 (256) or 85 (512) points
-    constexpr int HB = NT >= 512 ? 3 : 6;      // rows up to 128 points
     StepArgs<A> p;
     p.x = x; p.old = old; p.out = out; p.veff = static_cast<const A *>(veff);
     p.ldx = ldx; p.ldo = ldo; p.ldout = ldout;
@@ -1168,16 +1164,7 @@ void launch_step_rp(const StencilGeom &g, const void *x, long ldx, const void *o
             for (int q = 0; q < 2; ++q) p.ph[ax][sd][q] = (A)g.phase[ax][sd][q];
     const int blocks = ((p.nwork + 7) / 8) * 8;
     const size_t shm = 2 * sizeof(S) * ((size_t)pitch * (p.tyr + 2 * kMaxR) + NT);
-    const bool small_halo = 2 * kMaxR * g.nx <= NT * HS;
-    if (pitch == 64) {
-        if (small_halo) hipLaunchKernelGGL((k_stencil_step<S, kMaxR, RP, NT, HS, 64>), dim3(blocks), dim3(NT), shm, st, p);
-        else hipLaunchKernelGGL((k_stencil_step<S, kMaxR, RP, NT, HB, 64>), dim3(blocks), dim3(NT), shm, st, p);
-    } else if (pitch == 128) {
-        if (small_halo) hipLaunchKernelGGL((k_stencil_step<S, kMaxR, RP, NT, HS, 128>), dim3(blocks), dim3(NT), shm, st, p);
-        else hipLaunchKernelGGL((k_stencil_step<S, kMaxR, RP, NT, HB, 128>), dim3(blocks), dim3(NT), shm, st, p);
-    } else if constexpr (NT >= 512) {
-        hipLaunchKernelGGL((k_stencil_step<S, kMaxR, RP, NT, kLongHalo, 256>), dim3(blocks), dim3(NT), shm, st, p);
-    }
+    hipLaunchKernelGGL((k_stencil_step<S, kMaxR, RP, NT, kLongHalo, 256>), dim3(blocks), dim3(NT), shm, st, p);
 }
 
 // run width of the vector stencil for rows of nx points: 16-byte runs, else
@@ -1341,10 +1328,19 @@ void stencil_step(int e, const StencilGeom &g, const void *x, long ldx, const vo
     dispatch(e, [&](auto t) {
         using S = decltype(t);
         constexpr int B = base_rp<S>();
-        if (!g.orth || Tr<S>::C) {
+        if constexpr (!Tr<S>::C) {
+            if (g.orth && cfg.vec &&
+                launch_vec_modes<S, S>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg, st, coef))
+                return;
+        }
+        if (!g.orth || Tr<S>::C || tile_pitch(g.nx) < 256) {
             // one point per thread (stencil_points.hpp); the rows each of the
             // four shapes takes are those of its tile, points per thread
-            // included, as the tuner lists them
+            // included, as the tuner lists them.  Real orthogonal rows of
+            // more than 116 points keep the scalar body below, whose threads
+            // hold several points: 200 x 40 x 40 x 60 double 183 us against
+            // 216 us, bands of two rows beside 12 halo rows; 25 x 27 x 29 x
+            // 1600 double takes 209 us here and 311 us there.
             const int nt = cfg.nt >= 512 ? 512 : 256;
             const int rp = std::max(1, (g.orth ? B : B / 4) / (cfg.rp_div >= 2 ? 2 : 1));
             PointShape sh;
@@ -1355,19 +1351,11 @@ void stencil_step(int e, const StencilGeom &g, const void *x, long ldx, const vo
             return;
         }
         if constexpr (!Tr<S>::C) {
-            if (cfg.vec && launch_vec_modes<S, S>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg, st, coef))
-                return;
-            if (cfg.nt >= 512) {
-                if (cfg.rp_div >= 2)
-                    launch_step_rp<S, B / 2, 512>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
-                else
-                    launch_step_rp<S, B, 512>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
-            } else {
-                if (cfg.rp_div >= 2)
-                    launch_step_rp<S, B / 2, 256>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
-                else
-                    launch_step_rp<S, B, 256>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
-            }
+            if (cfg.nt < 512) fail(8, "grid rows longer than the fused stencil kernel's tile are not supported");
+            if (cfg.rp_div >= 2)
+                launch_step_rp<S, B / 2, 512>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
+            else
+                launch_step_rp<S, B, 512>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
         }
     });
 }
@@ -1440,14 +1428,11 @@ struct BatchPlan {
     int e = 0, n = 0;
     void *recs = nullptr;
     struct SGroup {
-        int kind = 0;             // 0 real orthogonal, 1 complex or non-orthogonal, 2 / 3 real orthogonal 16- / 8-byte runs
-        int W = 64;
+        bool points = true;       // one point per thread, else real orthogonal long rows
         int *items = nullptr;
         int nitems = 0;
         int max_tyr = 0;
-        bool small_halo = true;   // fewer halo slots per thread suffice for every unit of the group
-        int nt = 256;             // threads per workgroup (512 for long rows)
-        bool nonorth = false;     // kind 1: cell, and launch shape of its units (rows per band differ)
+        bool nonorth = false;     // points: cell, and launch shape of its units (rows per band differ)
         PointShape shape;
     };
     struct NGroup {
@@ -1484,12 +1469,9 @@ T *dev_upload(const std::vector<T> &v, hipStream_t st)
     return d;
 }
 
-// points per thread of the batched stencil shapes (256 threads per group)
+// points per thread of batched long rows
 template <class S> constexpr int batch_rp_orth() { return base_rp<S>() / 2 > 0 ? base_rp<S>() / 2 : 1; }
-constexpr int kBatchNT = 256;
-// runs per thread of the batched run-vector kinds (two, for taller bands
-// and less halo, ran slower: more registers, fewer waves)
-constexpr int kBatchRuns = 1;
+
 template <class S>
 void build_batch(BatchPlan *P, const BatchUnit *units, int n, hipStream_t st)
 {
@@ -1497,58 +1479,29 @@ void build_batch(BatchPlan *P, const BatchUnit *units, int n, hipStream_t st)
     std::vector<BatchRec<A>> recs(n);
     // stencil groups by (orth, pitch, threads), nonlocal groups by npm
     std::vector<int> sgi(n), ngi(n, -1);
-    std::vector<int> kind(n), ntu(n, kBatchNT);
+    std::vector<char> points(n);
     std::vector<PointShape> shape(n);
     for (int u = 0; u < n; ++u) {
         const StencilGeom &g = units[u].g;
         if (g.nx + 2 * kMaxR > 256) fail(8, "grid rows longer than the fused stencil kernel's tile are not supported");
-        kind[u] = g.orth && !Tr<S>::C ? 0 : 1;
-        int W = tile_pitch(g.nx);
-        bool sh = 2 * kMaxR * g.nx <= kBatchNT * 3;
-        if (kind[u] == 1) {
-            if (!g.orth && W == 256 && sizeof(S) > 8)
+        const bool longrow = tile_pitch(g.nx) == 256;
+        points[u] = !g.orth || Tr<S>::C || !longrow;
+        if (points[u]) {
+            if (!g.orth && longrow && sizeof(S) > 8)
                 fail(8, "complex128 non-orthogonal grids with rows over 116 points are not supported");
             if (!point_shape_batch(P->e, g, shape[u]))
                 fail(8, "grid rows longer than the batched stencil kernel's tile are not supported");
-            W = shape[u].pitch;
-            ntu[u] = shape[u].nt;
-            sh = true;
-        } else if (W == 256) {
-            // long rows: 512 threads, a 256-point pitch and kLongHalo halo
-            // slots per thread, scalar bodies (no vector runs)
-            ntu[u] = 512;
-            sh = false;
-        }
-        if constexpr (!Tr<S>::C) {
-            // kind 2: 16-byte runs; kind 3: 8-byte runs of two floats for
-            // rows whose length is not a multiple of four
-            const BatchUnit &U = units[u];
-            auto try_vec = [&](int VW, int kd) {
-                const int XO = (kMaxR + VW - 1) / VW * VW;
-                const uintptr_t am = (uintptr_t)(VW * sizeof(S)) - 1;
-                auto al = [&](const void *ptr, long ld) {
-                    return (reinterpret_cast<uintptr_t>(ptr) & am) == 0 && ld % VW == 0;
-                };
-                const int lpr = (g.nx / VW + 15) / 16 * 16;
-                if (g.orth && g.nx % VW == 0 && g.nx + 2 * XO <= 128 && g.nx >= 2 * XO && lpr <= kBatchNT &&
-                    al(U.buf[0], U.ld[0]) && al(U.buf[1], U.ld[1]) && al(U.buf[2], U.ld[2]) && al(U.veff, 0)) {
-                    kind[u] = kd;
-                    W = g.nx + 2 * XO <= 64 ? 64 : 128;
-                    sh = 2 * kMaxR * lpr <= kBatchNT * 2;
-                    return true;
-                }
-                return false;
-            };
-            if (!try_vec(int(16 / sizeof(S)), 2) && sizeof(S) == 4) try_vec(2, 3);
         }
         int k = -1;
-        for (size_t i = 0; i < P->sg.size(); ++i)
-            if (P->sg[i].kind == kind[u] && P->sg[i].W == W && P->sg[i].small_halo == sh && P->sg[i].nt == ntu[u] &&
-                (kind[u] != 1 || (P->sg[i].nonorth == !g.orth && P->sg[i].shape.hp == shape[u].hp &&
-                                  P->sg[i].shape.wrapz == shape[u].wrapz)))
+        for (size_t i = 0; i < P->sg.size(); ++i) {
+            const PointShape &a = P->sg[i].shape, &b = shape[u];
+            if (P->sg[i].points == (bool)points[u] &&
+                (!points[u] || (P->sg[i].nonorth == !g.orth && a.pitch == b.pitch && a.nt == b.nt && a.hp == b.hp &&
+                                a.wrapz == b.wrapz)))
                 k = (int)i;
+        }
         if (k < 0) {
-            P->sg.push_back({kind[u], W, nullptr, 0, 0, sh, ntu[u], !g.orth, shape[u]});
+            P->sg.push_back({(bool)points[u], nullptr, 0, 0, !g.orth, shape[u]});
             k = (int)P->sg.size() - 1;
         }
         sgi[u] = k;
@@ -1585,25 +1538,14 @@ void build_batch(BatchPlan *P, const BatchUnit *units, int n, hipStream_t st)
         r.q = operator_args<A>(g);
         StepArgs<A> &p = r.q.b;
         p.ncol = U.ncol;
-        if (kind[u] == 2 || kind[u] == 3) {
-            // kBatchRuns runs per thread, band rows at lane multiples of 16
-            const int VW = kind[u] == 3 ? 2 : int(16 / sizeof(S));
-            p.lpr = (g.nx / VW + 15) / 16 * 16;
-            const int rpb = kBatchRuns * kBatchNT / p.lpr;
-            const int nb = (g.ny + rpb - 1) / rpb;
-            p.tyr = (g.ny + nb - 1) / nb;
-        } else if (kind[u] == 1) {
-            p.lpr = 0;
+        p.lpr = 0;
+        if (points[u]) {
             p.tyr = shape[u].tyr;
         } else {
-            const int nt = ntu[u];
-            const long pts = (long)nt * batch_rp_orth<S>();
-            const int hslots = nt == 512 ? kLongHalo : 6;
-            if (g.nx > pts || 2 * kMaxR * g.nx > nt * hslots)
+            const long pts = 512L * batch_rp_orth<S>();
+            if (g.nx > pts || 2 * kMaxR * g.nx > 512 * kLongHalo)
                 fail(8, "grid rows longer than the batched stencil kernel's tile are not supported");
-            p.lpr = 0;
-            const int max_rows = step_max_rows<S>(P->sg[sgi[u]].W, nt);
-            if (max_rows < 1) fail(8, "grid rows longer than the batched stencil kernel's tile are not supported");
+            const int max_rows = step_max_rows<S>(256, 512);
             int nb = (int)(((long)g.nx * g.ny + pts - 1) / pts);
             nb = std::max(1, std::min(nb, g.ny));
             p.tyr = (g.ny + nb - 1) / nb;
@@ -1702,34 +1644,6 @@ void build_batch(BatchPlan *P, const BatchUnit *units, int n, hipStream_t st)
     P->beta_bytes = (beta_off * sizeof(S) + 255) / 256 * 256;
     hip_check(hipMalloc(&P->beta, std::max<size_t>(1, 2 * P->beta_bytes)), "hipMalloc");
     hip_check(hipStreamSynchronize(st), "batch upload");
-}
-
-template <class S, int W, int HP>
-void launch_stencil_batch(const BatchPlan *P, const BatchPlan::SGroup &G, const void *coef, int ix, int iold,
-                          int iout, hipStream_t st)
-{
-    const int blocks = ((G.nitems + 7) / 8) * 8;
-    const auto *recs = static_cast<const BatchRec<S> *>(P->recs);
-    const S *cf = static_cast<const S *>(coef);
-    auto go = [&](auto kern, int nt, size_t shm) {
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(nt), shm, st, recs, G.items, G.nitems, cf, ix, iold, iout);
-    };
-    if constexpr (W == 256) {
-        // long rows: 512 threads, scalar body
-        const size_t shm = 2 * sizeof(S) * ((size_t)W * (G.max_tyr + 2 * kMaxR) + 512);
-        go(k_stencil_batch<S, kMaxR, batch_rp_orth<S>(), 512, kLongHalo, W, 0>, 512, shm);
-    } else if (G.kind == 2 || G.kind == 3) {
-        // vector kinds: halo slots counted in runs (2 or 3 per thread)
-        constexpr int HV = HP == 3 ? 2 : 3;
-        const int VW = G.kind == 3 ? 2 : int(16 / sizeof(S));
-        const size_t shm = 2 * sizeof(S) * ((size_t)W * (G.max_tyr + 2 * kMaxR) + kBatchNT * VW);
-        if (G.kind == 2) go(k_stencil_batch<S, kMaxR, kBatchRuns, kBatchNT, HV, W, 2>, kBatchNT, shm);
-        else if constexpr (sizeof(S) == 4)
-            go(k_stencil_batch<S, kMaxR, kBatchRuns, kBatchNT, HV, W, 3>, kBatchNT, shm);
-    } else {
-        const size_t shm = 2 * sizeof(S) * ((size_t)W * (G.max_tyr + 2 * kMaxR) + kBatchNT);
-        go(k_stencil_batch<S, kMaxR, batch_rp_orth<S>(), kBatchNT, HP, W, 0>, kBatchNT, shm);
-    }
 }
 
 template <class S, int NPM>
@@ -1833,20 +1747,15 @@ void batch_step(BatchPlan *P, int step, int ix, int iold, int iout, bool first, 
                               G.update ? beta[step & 1] : beta[0], cf, ix, st);
         }
         for (const auto &G : P->sg) {
-            if (G.kind == 1) {
+            if (G.points) {
                 points_batch(P->e, P->recs, G.items, G.nitems, G.nonorth, cf, ix, iold, iout, G.shape, st);
                 continue;
             }
             if constexpr (!Tr<S>::C) {
-                if (G.W == 64) {
-                    if (G.small_halo) launch_stencil_batch<S, 64, 3>(P, G, cf, ix, iold, iout, st);
-                    else launch_stencil_batch<S, 64, 6>(P, G, cf, ix, iold, iout, st);
-                } else if (G.W == 256) {
-                    launch_stencil_batch<S, 256, kLongHalo>(P, G, cf, ix, iold, iout, st);
-                } else {
-                    if (G.small_halo) launch_stencil_batch<S, 128, 3>(P, G, cf, ix, iold, iout, st);
-                    else launch_stencil_batch<S, 128, 6>(P, G, cf, ix, iold, iout, st);
-                }
+                const size_t shm = 2 * sizeof(S) * (256 * (size_t)(G.max_tyr + 2 * kMaxR) + 512);
+                hipLaunchKernelGGL((k_stencil_batch<S, batch_rp_orth<S>()>), dim3((G.nitems + 7) / 8 * 8), dim3(512),
+                                   shm, st, static_cast<const BatchRec<S> *>(P->recs), G.items, G.nitems,
+                                   static_cast<const S *>(cf), ix, iold, iout);
             }
         }
         for (const auto &G : P->ng) {

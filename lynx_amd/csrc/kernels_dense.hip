@@ -22,7 +22,10 @@ typedef double double4v __attribute__((ext_vector_type(4)));
 template <class S>
 __device__ __forceinline__ S *unit_of(const NarrowBlocks &b, long ld, int u)
 {
-    return b.table ? static_cast<S *>(b.table[u]) : static_cast<S *>(b.base) + (long)u * b.stride;
+    // (the address space of a pointer read from memory is not known otherwise)
+    typedef __attribute__((address_space(1))) S *G;
+    return (S *)(G)reinterpret_cast<unsigned long>(b.table ? static_cast<S *>(b.table[u])
+                                                           : static_cast<S *>(b.base) + (long)u * b.stride);
 }
 
 // -------------------------------------------------------------------- Gram --

@@ -193,9 +193,9 @@ __global__ void __launch_bounds__(1024) k_nl_tile_batch(const BatchRec<typename 
     const int u = item_unit[w];
     const BatchRec<typename Tr<S>::A> &r = recs[u];
     const int lb = w - r.g_item0;
-    nl_tile_body<S, NPM, MODE, S>(r.nl, beta_in + r.beta_off, beta_out + r.beta_off,
-                                  reinterpret_cast<S *>(const_cast<void *>(r.buf[iy])), r.ld[iy], r.ncol, coef[3 * u],
-                                  lb % r.nl.n_atom, lb / r.nl.n_atom);
+    nl_tile_body<S, NPM, MODE, S>(global_args(r.nl), beta_in + r.beta_off, beta_out + r.beta_off,
+                                  global_ptr(reinterpret_cast<S *>(const_cast<void *>(r.buf[iy]))), r.ld[iy], r.ncol,
+                                  coef[3 * u], lb % r.nl.n_atom, lb / r.nl.n_atom);
 }
 
 template <class F>

@@ -45,20 +45,22 @@ bool point_shape(int e, const StencilGeom &g, int max_threads, int nzch, PointSh
 }
 
 // The cost of a shape per point: idle lanes, halo rows (a tenth of an own
-// row's cost each) and, above 256 threads, fewer workgroups to a CU to hide
-// each other's barriers.  Measured at 24^3 x 1344 complex64: 8 rows in 192
-// threads 176 us, 12 in 320 249 us, 4 in 128 (a quarter of them idle) 218 us,
-// 24 in 576 280 us; at 32^3 x 400: 8 rows in 256 136 us, 4 in 128 160 us,
-// 16 in 512 189 us.
+// row's cost each) and, with 512 threads, fewer workgroups to a CU to hide
+// each other's barriers; 320 to 448 threads leave too many wave slots empty.
+// Measured (rows / threads): 24^3 x 1344 complex64 skew 8/192 176 us, 12/320
+// 249, 4/128 218; 32^3 x 400 8/256 136, 4/128 160, 16/512 189; double 30^3 x
+// 1600 6/192 281, 8/256 289, 10/320 354, 15/512 312; 40^3 x 600 6/256 247,
+// 4/192 270, 8/320 288; 50^3 x 300 5/256 246, 10/512 234, 7/384 314; 100 x 60
+// x 60 x 60 5/512 191, 2/256 218, 3/320 250.
 bool point_shape_batch(int e, const StencilGeom &g, PointShape &out)
 {
     double best = 0;
-    for (int budget : {128, 192, 256, 320, 384, 448, 512}) {
+    for (int budget : {128, 192, 256, 512}) {
         PointShape s;
         if (!point_shape(e, g, budget, 1, s)) continue;
         const int nb = (g.ny + s.tyr - 1) / s.tyr;
         double cost = (double)nb * s.nt / ((double)g.nx * g.ny) * (1.0 + 0.12 * 2 * kMaxR / s.tyr);
-        if (s.nt > 256) cost *= 1.0 + (s.nt - 256) / 400.0;
+        if (s.nt > 256) cost *= 1.64;
         if (best == 0 || cost < best) {
             best = cost;
             out = s;

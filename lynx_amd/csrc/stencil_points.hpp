@@ -59,6 +59,10 @@ struct PointLoads {
 // end planes' partial sums in memory, the same step took 297 us; complex128
 // 553 us, now 305 us (892 MB: 2.9 TB/s).  Alone: 48^3 x 64 double skew 93 ->
 // 69 us, 40^3 x 48 complex128 orthogonal 75 -> 47 us.
+// Real orthogonal blocks that the run-vector kernel does not take, and all of
+// them in batches: 25 x 27 x 29 x 1600 double 311 -> 209 us against several
+// points per thread; batches of 24..40^3 frames, 15.3 M points in all, step of
+// double 600 us as 16-byte runs, now 568 us (all launches of a step).
 template <class S, bool NONORTH, bool WRAPZ, int HP, int W>
 __device__ __forceinline__ void stencil_points_body(const NonorthArgs<typename Tr<S>::A> &q,
                                                     const StepIO<typename Tr<S>::A> io, const int w)
@@ -84,9 +88,10 @@ __device__ __forceinline__ void stencil_points_body(const NonorthArgs<typename T
     const int z0 = zc * p.zch;
     const int z1 = min(z0 + p.zch, nz);
     const int nxny = nx * ny;
-    const S *__restrict__ X = reinterpret_cast<const S *>(io.x) + (long)col * io.ldx;
-    const S *__restrict__ O = reinterpret_cast<const S *>(io.old) + (long)col * io.ldo;
-    S *__restrict__ Y = reinterpret_cast<S *>(io.out) + (long)col * io.ldout;
+    const S *__restrict__ X = global_ptr(reinterpret_cast<const S *>(io.x)) + (long)col * io.ldx;
+    const S *__restrict__ O = global_ptr(reinterpret_cast<const S *>(io.old)) + (long)col * io.ldo;
+    S *__restrict__ Y = global_ptr(reinterpret_cast<S *>(io.out)) + (long)col * io.ldout;
+    const A *__restrict__ Vf = global_ptr(p.veff);
     const bool has_old = io.old != nullptr && io.b != A(0);   // no Y_(k-2) stream without a buffer
 
     // the owned point; lanes beyond the band repeat its last one (and write
@@ -152,7 +157,7 @@ __device__ __forceinline__ void stencil_points_body(const NonorthArgs<typename T
             for (int h = 0; h < HP; ++h) L.halo[h] = ld_at(Xz, hoff[h]);
         }
         if (has_old) L.old = ld_at(O + max(f - R, WRAPZ ? R : z0) * nxny, off);
-        L.v = ld_at(p.veff + min(max(f, z0), z1 - 1) * nxny, off);
+        L.v = ld_at(Vf + min(max(f, z0), z1 - 1) * nxny, off);
     };
 
     // acc[j]: -2 (H - s) x at output plane f - R + j, so H x = -acc / 2

@@ -1,5 +1,5 @@
-"""The one-point-per-thread stencil step (complex blocks and non-orthogonal
-cells) at the edges of its launch shapes, against the oracle: rows shorter
+"""The one-point-per-thread stencil step (complex blocks, non-orthogonal cells,
+and real orthogonal ones without the run-vector kernel) at the edges of its launch shapes, against the oracle: rows shorter
 than two ghost widths (both copies of a point), fewer than 12 planes (no march
 once around z) and z-chunks, rows at the limits of each LDS pitch, a band of
 one row, grids smaller than a workgroup.  H applies and a filter (the
@@ -44,8 +44,6 @@ def test_points_step_matches_oracle(n, skew):
     lc = lo + 0.3 * (hi - lo)
     for dt in DTYPES:
         cplx = np.dtype(dt).kind == "c"
-        if not skew and not cplx:
-            continue
         single = np.dtype(dt).itemsize == (8 if cplx else 4)
         k = s.kpt if cplx else (0.0, 0.0, 0.0)
         op.set_kpoint(k)
