@@ -643,7 +643,7 @@ void gram(lynx_ctx *c, int e, const void *A, long lda, const void *B, long ldb, 
         const int ns = gpu::gram_f64_splits(nd, n);
         void *W = c->gwork.get((size_t)ns * n * n * sizeof(double));
         const int used = gpu::gram_f64(static_cast<const double *>(A), lda, static_cast<const double *>(B), ldb, nd,
-                                       n, static_cast<double *>(W), ns, true, c->stream);
+                                       n, static_cast<double *>(W), ns, c->stream);
         gpu::gram_reduce(e, W, used, n, alpha, C, c->stream);
         return;
     }

@@ -216,82 +216,90 @@ __global__ void __launch_bounds__(kThreads) k_gram_bf16x3(const float *__restric
 // ------------------------------------------------------------- FP64 Gram --
 // C = A^T B for FP64 blocks on v_mfma_f64_16x16x4f64 (lane l supplies
 // A[l % 16][l / 16] and B[l / 16][l % 16] and holds D[l / 16 + 4 v][l % 16],
-// v = 0..3; checked on gfx950).  Same decomposition as k_gram_bf16x3: one
-// workgroup per (tile pair, K chunk); for A^T A, or a product whose
-// Hermitian part is wanted (upper), only the tiles on and above the
-// diagonal, their upper entries written to both halves; one FP64 partial
-// product per chunk summed in a fixed order by gram_reduce.  A workgroup of four waves owns a
-// 128 x 128 tile; wave w takes the 64 x 64 quarter (w / 2, w % 2), 4 x 4
-// products per 4-deep step, each fragment read once from LDS and used four
-// times.  Per 32-deep block the tile's 128 columns of A and of B are staged
-// in LDS with k contiguous (33 doubles per column, so the 16 lanes reading
-// one k of 16 columns hit distinct banks); the next block's loads are in
-// flight while the current block's products run.
-constexpr int kDT = 128;          // C tile edge
-constexpr int kDKB = 32;          // K rows per LDS block
-constexpr int kDP = kDKB + 1;     // doubles per LDS column
+// v = 0..3; checked on gfx950), for A^T A or a product whose Hermitian part
+// is wanted: only 16 x 16 products on and above the diagonal, their upper
+// entries written to both halves; one partial product per K chunk summed in a
+// fixed order by gram_reduce.
+//
+// A workgroup of four waves owns a 96 x 96 tile of one chunk; wave w takes
+// the 48 x 48 quarter (w / 2, w % 2), 3 x 3 products per 4-deep step; a
+// quarter below the diagonal or beyond the last column is left out, and the
+// wave's SIMD runs those of the other two workgroups of the CU.  Per 16-deep
+// block the tile's columns of A and of B are staged in LDS; 8 lanes load 128
+// contiguous bytes of a column, the next block's loads are in flight while
+// the current block's products run, and a column pitch of 18 doubles lets 32
+// lanes (16 columns, two k) read distinct banks.  32-deep blocks need more
+// registers than three workgroups per CU leave.
+//
+// Bound by the matrix cores: 480 columns of 90^3 points 3.4 ms (50 TFLOP/s of
+// the half product), with 128 x 128 tiles and 32-deep blocks, one workgroup
+// per CU, 5.9 ms (5.4 ms A = B); 160 of 60^3 0.22 ms.  Fragments straight from
+// memory, without LDS or barriers: 5.2-5.6 ms.
+constexpr int kDT = 96;           // C tile edge
+constexpr int kDW = kDT / 32;     // 16 x 16 products per wave and direction
+constexpr int kDKB = 16;          // K rows per LDS block
+constexpr int kDP = kDKB + 2;     // doubles per LDS column
+constexpr int kDR = kDKB / 2;     // lanes that load one column's block, 16 bytes each
+constexpr int kDL = kDT * kDR / 256;   // loads per thread, block and operand
 typedef double double4v __attribute__((ext_vector_type(4)));
 
-// This thread's share of a 32-deep block of a 128-column tile: 16
-// consecutive K rows (from k0 + koff, masked by kend and the column count)
-// of column c = t / 2.
 struct DSlab {
-    double v[kDKB / 2];
+    double2 v[kDL];
 };
 
+// rows k0 + 2 (t % kDR), + 1 of columns col0 + t / kDR + 256 q / kDR, zero
+// beyond kend and the column count
 __device__ inline void load_dslab(const double *__restrict__ X, long ldx, long k0, long kend, int col0, int N, int t,
                                   DSlab &s)
 {
-    const int c = t >> 1;
-    const int koff = (t & 1) * (kDKB / 2);
-    const int gc = col0 + c;
-    const long r0 = k0 + koff;
-    if (gc < N && r0 + kDKB / 2 <= kend) {
-        const double2 *p = reinterpret_cast<const double2 *>(X + (long)gc * ldx + r0);
+    const long r = k0 + 2 * (t % kDR);
+    const int c = col0 + t / kDR;
+    const double *p = X + (long)c * ldx + r;
 #pragma unroll
-        for (int q = 0; q < kDKB / 4; ++q) {
-            const double2 f = p[q];
-            s.v[2 * q] = f.x;
-            s.v[2 * q + 1] = f.y;
+    for (int q = 0; q < kDL; ++q) {
+        s.v[q] = make_double2(0.0, 0.0);
+        if (c + 256 / kDR * q < N) {
+            if (r + 1 < kend) s.v[q] = *reinterpret_cast<const double2 *>(p);
+            else if (r < kend) s.v[q].x = p[0];
         }
-    } else {
-#pragma unroll
-        for (int i = 0; i < kDKB / 2; ++i) s.v[i] = (gc < N && r0 + i < kend) ? X[(long)gc * ldx + r0 + i] : 0.0;
+        p += 256 / kDR * ldx;
     }
 }
 
 __device__ inline void store_dslab(const DSlab &s, double *lds, int t)
 {
-    double *d = lds + (t >> 1) * kDP + (t & 1) * (kDKB / 2);
 #pragma unroll
-    for (int i = 0; i < kDKB / 2; ++i) d[i] = s.v[i];
+    for (int q = 0; q < kDL; ++q)
+        *reinterpret_cast<double2 *>(lds + (t / kDR + 256 / kDR * q) * kDP + 2 * (t % kDR)) = s.v[q];
 }
 
-__global__ void __launch_bounds__(256) k_gram_f64(const double *__restrict__ A, long lda,
+__global__ void __launch_bounds__(256, 3) k_gram_f64(const double *__restrict__ A, long lda,
                                                   const double *__restrict__ B, long ldb, long K, int N, long kch,
-                                                  int tiles_n, int same, int upper, int pairs, int items,
-                                                  int per_xcd, double *__restrict__ part)
+                                                  int tiles_n, int same, int pairs, int items, int per_xcd,
+                                                  double *__restrict__ part)
 {
     const int item = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
     if (item >= items) return;
     const int chunk = item / pairs, pair = item % pairs;
-    __shared__ double sA[kDT * kDP], sB[kDT * kDP];
+    __shared__ __align__(16) double sA[kDT * kDP], sB[kDT * kDP];
     const int t = threadIdx.x, w = t >> 6, l = t & 63;
     int tm, tn;
-    tile_of(pair, tiles_n, upper, tm, tn);
+    tile_of(pair, tiles_n, 1, tm, tn);
     const int m0 = tm * kDT, n0 = tn * kDT;
     const long kbeg = (long)chunk * kch, kend = std::min(K, kbeg + kch);
     const bool one = same && tm == tn;          // B's tile is A's
     const double *sb = one ? sA : sB;
     const double *Bsrc = same ? A : B;
     const long ldbs = same ? lda : ldb;
-    const int wm = (w >> 1) * 64, wn = (w & 1) * 64;
+    const int wm = (w >> 1) * (kDT / 2), wn = (w & 1) * (kDT / 2);
     const int lr = l & 15, lk = l >> 4;
-    double4v acc[4][4];
+    // whether any product of this wave is wanted
+    const bool work = m0 + wm <= n0 + wn && n0 + wn < N;
+    double4v acc[kDW][kDW];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < kDW; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = double4v{0.0, 0.0, 0.0, 0.0};
+        for (int j = 0; j < kDW; ++j) acc[i][j] = double4v{0.0, 0.0, 0.0, 0.0};
     DSlab xa, xb;
     if (kbeg < kend) {
         load_dslab(A, lda, kbeg, kend, m0, N, t, xa);
@@ -305,44 +313,37 @@ __global__ void __launch_bounds__(256) k_gram_f64(const double *__restrict__ A, 
             load_dslab(A, lda, k0 + kDKB, kend, m0, N, t, xa);
             if (!one) load_dslab(Bsrc, ldbs, k0 + kDKB, kend, n0, N, t, xb);
         }
+        const double *pa = sA + (wm + lr) * kDP + lk, *pb = sb + (wn + lr) * kDP + lk;
+        if (work) {
 #pragma unroll
-        for (int ks = 0; ks < kDKB; ks += 4) {
-            double a[4], b[4];
+            for (int ks = 0; ks < kDKB; ks += 4) {
+                double a[kDW], b[kDW];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = sA[(wm + 16 * i + lr) * kDP + ks + lk];
+                for (int i = 0; i < kDW; ++i) a[i] = pa[16 * i * kDP + ks];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = sb[(wn + 16 * j + lr) * kDP + ks + lk];
+                for (int j = 0; j < kDW; ++j) b[j] = pb[16 * j * kDP + ks];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+                for (int i = 0; i < kDW; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
+                    for (int j = 0; j < kDW; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
+            }
         }
         __syncthreads();
     }
     double *P = part + (size_t)chunk * N * N;
-    // upper: the tile's entries above the diagonal are mirrored below it;
-    // a diagonal tile of a non-symmetric product keeps its upper half only
-    const bool mirror = upper && tm != tn;
-    const bool diag_upper = upper && !same && tm == tn;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < kDW; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < kDW; ++j) {
+            if (!work) continue;
             const int n = n0 + wn + 16 * j + lr;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int m = m0 + wm + 16 * i + lk + 4 * v;
-                if (m < N && n < N) {
-                    if (diag_upper) {
-                        if (m <= n) {
-                            P[m + (size_t)n * N] = acc[i][j][v];
-                            P[n + (size_t)m * N] = acc[i][j][v];
-                        }
-                    } else {
-                        P[m + (size_t)n * N] = acc[i][j][v];
-                        if (mirror) P[n + (size_t)m * N] = acc[i][j][v];
-                    }
+                if (m <= n && n < N) {
+                    P[m + (size_t)n * N] = acc[i][j][v];
+                    P[n + (size_t)m * N] = acc[i][j][v];
                 }
             }
         }
@@ -566,7 +567,9 @@ int gram_f64_splits(long K, int N)
 {
     const int tiles = (N + kDT - 1) / kDT;
     const int pairs = tiles * (tiles + 1) / 2;
-    const long want = std::max(1L, (768L + pairs - 1) / pairs);
+    // one round of the three workgroups that a CU holds: 780 items in 768
+    // slots took 4.4 ms, 765 take 3.4 ms (480 columns of 90^3 points)
+    const long want = std::max(1L, 768L / pairs);
     return (int)std::max(1L, std::min(want, (K + kDKB - 1) / kDKB));
 }
 
@@ -577,20 +580,19 @@ bool gram_f64_fits(const double *A, long lda, const double *B, long ldb)
 }
 
 int gram_f64(const double *A, long lda, const double *B, long ldb, long K, int N, double *part, int nsplit,
-             bool sym, hipStream_t st)
+             hipStream_t st)
 {
     if (N < 1 || K < 1 || nsplit < 1) throw std::runtime_error("gram_f64: empty product");
     if (!gram_f64_fits(A, lda, B, ldb)) throw std::runtime_error("gram_f64: columns must be 16-byte aligned");
     const int tiles = (N + kDT - 1) / kDT;
     const int same = A == B && lda == ldb ? 1 : 0;
-    const int upper = sym || same ? 1 : 0;
-    const int pairs = upper ? tiles * (tiles + 1) / 2 : tiles * tiles;
+    const int pairs = tiles * (tiles + 1) / 2;
     // chunk length: a multiple of the LDS block, so 16-byte loads stay aligned
     long kch = (K + nsplit - 1) / nsplit;
     kch = (kch + kDKB - 1) / kDKB * kDKB;
     const int used = (int)((K + kch - 1) / kch);
     const int items = pairs * used, per_xcd = (items + 7) / 8;
-    k_gram_f64<<<8 * per_xcd, 256, 0, st>>>(A, lda, B, ldb, K, N, kch, tiles, same, upper, pairs, items, per_xcd,
+    k_gram_f64<<<8 * per_xcd, 256, 0, st>>>(A, lda, B, ldb, K, N, kch, tiles, same, pairs, items, per_xcd,
                                             part);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) throw std::runtime_error(std::string("k_gram_f64: ") + hipGetErrorString(e));
