@@ -726,6 +726,15 @@ void rotate(lynx_ctx *c, int e, const void *A, long lda, const void *Q, int n, v
     }
 }
 
+// X <- X R for the upper triangular R in c->s1 where the triangular kernel
+// takes the block, else false.
+bool rotate_upper(lynx_ctx *c, int e, void *X, long ldx, int n)
+{
+    if (e != gpu::F64 || gpu::narrow_fits(e, n) || !gpu::rotate_upper_f64_fits(ldx, n)) return false;
+    gpu::rotate_upper_f64((double *)X, ldx, c->nd, c->s1.as<double>(), n, c->stream);
+    return true;
+}
+
 void *block(DevBuf &b, int e, long ld, int ncol) { return b.get((size_t)ld * ncol * gpu::elem_size(e)); }
 
 // ------------------------------------------------------- dense FP64 steps --
@@ -1317,9 +1326,11 @@ lynx_status lynx_orthogonalize(lynx_ctx *ctx, int dtype, void *x, int ld, int nc
             HIP_OK(hipMemcpy2DAsync(dx, nd * es, x, ldx * es, nd * es, ncol, hipMemcpyHostToDevice, ctx->stream));
         }
         cholesky_inverse(ctx, dtype, dx, ldd, ncol);
-        void *tmp = block(ctx->wB, dtype, padded_ld(nd), ncol);
-        rotate(ctx, dtype, dx, ldd, ctx->s1.p, ncol, tmp, padded_ld(nd));
-        gpu::copy_cols(dtype, tmp, padded_ld(nd), dx, ldd, nd, ncol, ctx->stream);
+        if (!rotate_upper(ctx, dtype, dx, ldd, ncol)) {
+            void *tmp = block(ctx->wB, dtype, padded_ld(nd), ncol);
+            rotate(ctx, dtype, dx, ldd, ctx->s1.p, ncol, tmp, padded_ld(nd));
+            gpu::copy_cols(dtype, tmp, padded_ld(nd), dx, ldd, nd, ncol, ctx->stream);
+        }
         if (mem != LYNX_MEM_DEVICE)
             HIP_OK(hipMemcpy2DAsync(x, ldx * es, dx, nd * es, nd * es, ncol, hipMemcpyDeviceToHost, ctx->stream));
         HIP_OK(hipStreamSynchronize(ctx->stream));
@@ -1501,9 +1512,11 @@ lynx_status lynx_chefsi_solve(lynx_ctx *ctx, int dtype, void *psi, int ld, int n
         // a8: Y = p_m(H) psi -> B
         filter(ctx, dtype, P, ldP, B, ldw, C, ldw, nband, degree, lambda_c, eig_min, eig_max);
         timing_end(ctx);
-        // a9: C = B R^-1 with dV B^H B = R^H R
+        // a9: C = B R^-1 with dV B^H B = R^H R (C takes B's place where it
+        // is formed in place)
         cholesky_inverse(ctx, dtype, B, ldw, nband);
-        rotate(ctx, dtype, B, ldw, ctx->s1.p, nband, C, ldw);
+        if (rotate_upper(ctx, dtype, B, ldw, nband)) std::swap(B, C);
+        else rotate(ctx, dtype, B, ldw, ctx->s1.p, nband, C, ldw);
         // a10: Hs = dV C^H H C (B <- H C)
         apply_op(ctx, dtype, C, ldw, nullptr, 0, B, ldw, nband, 1.0, 0.0, 0.0);
         void *H = ctx->s2.get((size_t)nband * nband * es);

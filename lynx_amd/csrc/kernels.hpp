@@ -135,6 +135,11 @@ int gram_f64(const double *A, long lda, const double *B, long ldb, long K, int N
              hipStream_t st);
 int gram_f64_splits(long K, int N);
 bool gram_f64_fits(const double *A, long lda, const double *B, long ldb);
+// X (nd x N) <- X R in place for a real FP64 block and an upper triangular R
+// (N x N, ld N, zeros below the diagonal) (kernels_mfma.hip).  fits: its
+// 32-bit offsets reach.
+bool rotate_upper_f64_fits(long ld, int N);
+void rotate_upper_f64(double *X, long ld, long nd, const double *R, int N, hipStream_t st);
 // Split-BF16x3 rotation on the matrix cores (kernels_mfma.hip): C (M x N) =
 // A (M x K) Q (K x N) for a real FP32 block A (column-major, ld lda) and an
 // FP64 Q (ld ldq), both split into bfloat16 hi + lo, hi.hi + hi.lo + lo.hi
