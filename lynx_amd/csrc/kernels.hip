@@ -219,6 +219,14 @@ __global__ void __launch_bounds__(NT) k_stencil_step(StepArgs<typename Tr<S>::A>
 // read per offset.  This cuts the LDS instructions per point by about 2.5x
 // and makes every global access a dwordx4 (dwordx2).  Requires nx % VW == 0
 // and columns aligned to the run size.
+//
+// What bounds it: latency, at two to three waves per SIMD (f32: vector
+// instructions 45 %, LDS 40 %, memory 70 % of the time).  The two runs of a
+// thread are adjacent rows, so 12 LDS reads serve the y terms of both instead
+// of 24, and the sums are formed outside the branch of the store: inside it
+// every LDS value lived until the branch (198 registers, now 160: three waves
+// per SIMD instead of two).  90^3 x 480 float 1267 -> 1050 us a step, 60^3 x
+// 160 bfloat16 116 -> 93 us, double 236 -> 207 us.
 template <class S, int VW, int RV, int HP>
 struct VecLoads {
     VRun<S, VW> front[RV];
@@ -226,6 +234,39 @@ struct VecLoads {
     VRun<S, VW> v[RV];
     VRun<S, VW> halo[HP];
 };
+
+// lap[r] += sum_k c[k] (row y_r + k, row y_r - k) for the RV runs of a thread in
+// adjacent rows y_0 + r: each row is read once from LDS (L: run 0's element)
+// and joins every run within R of it; own: the runs themselves.
+template <class S, int R, int RV, int W, int VW>
+__device__ __forceinline__ void add_rows(const S *L, const S *c, const VRun<S, VW> (&own)[RV],
+                                         VRun<S, VW> (&lap)[RV])
+{
+#pragma unroll
+    for (int k = 1; k <= R; ++k) {
+        // rows k below run 0 and k above the last run
+        const VRun<S, VW> dn = *reinterpret_cast<const VRun<S, VW> *>(L - k * W);
+        const VRun<S, VW> up = *reinterpret_cast<const VRun<S, VW> *>(L + (RV - 1 + k) * W);
+#pragma unroll
+        for (int r = 0; r < RV; ++r)
+#pragma unroll
+            for (int e = 0; e < VW; ++e) {
+                if (RV == 1) {
+                    lap[r].v[e] = fm(c[k], add(up.v[e], dn.v[e]), lap[r].v[e]);
+                    continue;
+                }
+                if (k + r <= R) lap[r].v[e] = fm(c[k + r], dn.v[e], lap[r].v[e]);
+                if (RV - 1 - r + k <= R) lap[r].v[e] = fm(c[RV - 1 - r + k], up.v[e], lap[r].v[e]);
+            }
+    }
+#pragma unroll
+    for (int r = 0; r < RV; ++r)
+#pragma unroll
+        for (int q = 0; q < RV; ++q)
+#pragma unroll
+            for (int e = 0; e < VW; ++e)
+                if (q != r) lap[r].v[e] = fm(c[q > r ? q - r : r - q], own[q].v[e], lap[r].v[e]);
+}
 
 template <class S, int R, int RV, int NT, int HP, int W, int VW, class T = S>
 __device__ __forceinline__ void stencil_vec_body(const StepArgs<S> &p, const StepIO<S> io, const int w)
@@ -259,7 +300,8 @@ __device__ __forceinline__ void stencil_vec_body(const StepArgs<S> &p, const Ste
     const int dummy = base + tid * VW;
     // owned runs: plane offset (element index), LDS index and x of the first
     // element (kNoX for lanes without a run, whose stores go to the dummy).
-    // Lane q takes run q % lpr of band row q / lpr; with lpr a multiple of 16
+    // Lane q takes run q % lpr of the RV band rows from RV (q / lpr) on, which
+    // share their y neighbours' LDS reads; with lpr a multiple of 16
     // no group of 16 lanes (one LDS cycle of 16-byte accesses) straddles two
     // rows, so row starts never collide in the same banks.
     constexpr int kNoX = -(1 << 20);
@@ -270,13 +312,15 @@ __device__ __forceinline__ void stencil_vec_body(const StepArgs<S> &p, const Ste
     bool qv[RV];
 #pragma unroll
     for (int r = 0; r < RV; ++r) {
-        const int q = tid + r * NT;
-        const int qy = q / lpr;
-        const int qr = q - qy * lpr;
+        const int q0 = tid / lpr;
+        const int qr = tid - q0 * lpr;
+        const int qy = RV * q0 + r;
         qv[r] = qy < rows && qr < runs;
         const int qx = qv[r] ? qr * VW : 0;
         const int qyy = qv[r] ? qy : 0;
         qoff[r] = qv[r] ? (y0 + qyy) * nx + qx : 0;
+        // a row above an odd band: the loaded run is the neighbour of run 0
+        if (r > 0 && !qv[r] && qv[0]) qoff[r] = (y0 + qy < ny ? y0 + qy : 0) * nx + qx0[0];
         qli[r] = qv[r] ? (qyy + R) * W + XO + qx : dummy;
         qx0[r] = qv[r] ? qx : kNoX;
     }
@@ -352,6 +396,7 @@ __device__ __forceinline__ void stencil_vec_body(const StepArgs<S> &p, const Ste
         for (int h = 0; h < HP; ++h) put(L, hli[h], hx0[h], cur.halo[h]);
         __syncthreads();
         T *Yz = Y + z * nxny;
+        VRun<S, VW> lap[RV], own[RV];
 #pragma unroll
         for (int r = 0; r < RV; ++r) {
             S xr[NXV * VW];
@@ -361,24 +406,30 @@ __device__ __forceinline__ void stencil_vec_body(const StepArgs<S> &p, const Ste
 #pragma unroll
                 for (int e = 0; e < VW; ++e) xr[j * VW + e] = t.v[e];
             }
-            S lap[VW];
 #pragma unroll
-            for (int e = 0; e < VW; ++e) lap[e] = diag * ring[r][R].v[e];
+            for (int e = 0; e < VW; ++e) lap[r].v[e] = diag * ring[r][R].v[e];
 #pragma unroll
-            for (int k = 1; k <= R; ++k) {
-                const VRun<S, VW> up = *reinterpret_cast<const VRun<S, VW> *>(L + qli[r] + k * W);
-                const VRun<S, VW> dn = *reinterpret_cast<const VRun<S, VW> *>(L + qli[r] - k * W);
+            for (int k = 1; k <= R; ++k)
 #pragma unroll
                 for (int e = 0; e < VW; ++e) {
-                    lap[e] = fm(p.c[0][k], add(xr[XO + e + k], xr[XO + e - k]), lap[e]);
-                    lap[e] = fm(p.c[1][k], add(up.v[e], dn.v[e]), lap[e]);
-                    lap[e] = fm(p.c[2][k], add(ring[r][R + k].v[e], ring[r][R - k].v[e]), lap[e]);
+                    lap[r].v[e] = fm(p.c[0][k], add(xr[XO + e + k], xr[XO + e - k]), lap[r].v[e]);
+                    lap[r].v[e] = fm(p.c[2][k], add(ring[r][R + k].v[e], ring[r][R - k].v[e]), lap[r].v[e]);
                 }
-            }
+            own[r] = ring[r][R];
+        }
+        add_rows<S, R, RV, W, VW>(L + qli[0], p.c[1], own, lap);
+        // computed by every lane: else all of it moves into the branch of the
+        // store, one run after the other, with every LDS value held till then
+#pragma unroll
+        for (int r = 0; r < RV; ++r)
+#pragma unroll
+            for (int e = 0; e < VW; ++e) asm volatile("" : "+v"(lap[r].v[e]));
+#pragma unroll
+        for (int r = 0; r < RV; ++r) {
             VRun<S, VW> res;
 #pragma unroll
             for (int e = 0; e < VW; ++e) {
-                const S hval = fm(cur.v[r].v[e] + io.s, ring[r][R].v[e], S(-0.5) * lap[e]);
+                const S hval = fm(cur.v[r].v[e] + io.s, ring[r][R].v[e], S(-0.5) * lap[r].v[e]);
                 res.v[e] = io.a * hval;
                 if (has_old) res.v[e] = fm(io.b, cur.old[r].v[e], res.v[e]);
             }
@@ -457,13 +508,15 @@ __device__ __forceinline__ void stencil_vacc_body(const StepArgs<S> &p, const St
     bool qv[RV];
 #pragma unroll
     for (int r = 0; r < RV; ++r) {
-        const int q = tid + r * NT;
-        const int qy = q / lpr;
-        const int qr = q - qy * lpr;
+        const int q0 = tid / lpr;
+        const int qr = tid - q0 * lpr;
+        const int qy = RV * q0 + r;
         qv[r] = qy < rows && qr < runs;
         const int qx = qv[r] ? qr * VW : 0;
         const int qyy = qv[r] ? qy : 0;
         qoff[r] = qv[r] ? (y0 + qyy) * nx + qx : 0;
+        // a row above an odd band: the loaded run is the neighbour of run 0
+        if (r > 0 && !qv[r] && qv[0]) qoff[r] = (y0 + qy < ny ? y0 + qy : 0) * nx + qx0[0];
         qli[r] = qv[r] ? (qyy + R) * W + XO + qx : dummy;
         qx0[r] = qv[r] ? qx : kNoX;
     }
@@ -543,6 +596,7 @@ __device__ __forceinline__ void stencil_vacc_body(const StepArgs<S> &p, const St
 #pragma unroll
             for (int h = 0; h < HP; ++h) put(L, hli[h], hx0[h], cur.halo[h]);
             __syncthreads();
+            VRun<S, VW> lap[RV];
 #pragma unroll
             for (int r = 0; r < RV; ++r) {
                 S xr[NXV * VW];
@@ -552,23 +606,18 @@ __device__ __forceinline__ void stencil_vacc_body(const StepArgs<S> &p, const St
 #pragma unroll
                     for (int e = 0; e < VW; ++e) xr[j * VW + e] = t.v[e];
                 }
-                S lap[VW];
 #pragma unroll
                 for (int e = 0; e < VW; ++e)
-                    lap[e] = fm(diag - S(2) * (cur.v[r].v[e] + io.s), cur.front[r].v[e], acc[r][R].v[e]);
+                    lap[r].v[e] = fm(diag - S(2) * (cur.v[r].v[e] + io.s), cur.front[r].v[e], acc[r][R].v[e]);
 #pragma unroll
-                for (int k = 1; k <= R; ++k) {
-                    const VRun<S, VW> up = *reinterpret_cast<const VRun<S, VW> *>(L + qli[r] + k * W);
-                    const VRun<S, VW> dn = *reinterpret_cast<const VRun<S, VW> *>(L + qli[r] - k * W);
+                for (int k = 1; k <= R; ++k)
 #pragma unroll
-                    for (int e = 0; e < VW; ++e) {
-                        lap[e] = fm(p.c[0][k], add(xr[XO + e + k], xr[XO + e - k]), lap[e]);
-                        lap[e] = fm(p.c[1][k], add(up.v[e], dn.v[e]), lap[e]);
-                    }
+                    for (int e = 0; e < VW; ++e)
+                        lap[r].v[e] = fm(p.c[0][k], add(xr[XO + e + k], xr[XO + e - k]), lap[r].v[e]);
                 }
+            add_rows<S, R, RV, W, VW>(L + qli[0], p.c[1], cur.front, lap);
 #pragma unroll
-                for (int e = 0; e < VW; ++e) acc[r][R].v[e] = lap[e];
-            }
+            for (int r = 0; r < RV; ++r) acc[r][R] = lap[r];
             buf ^= 1;
         }
         // z-neighbour terms of plane f for the outputs within R of it
@@ -1193,7 +1242,7 @@ bool launch_step_vec(const StencilGeom &g, const void *x, long ldx, const void *
         return false;
     const int runs = g.nx / VW;
     const int lpr = align ? (runs + 15) / 16 * 16 : runs;   // lanes per band row
-    const int rpb = NT * RV / lpr;                          // band rows per workgroup
+    const int rpb = NT / lpr * RV;                          // band rows per workgroup
     if (rpb < 1 || 2 * kMaxR * lpr > NT * HB || g.nx + 2 * XO > 128 || g.nx < 2 * XO) return false;
     StepArgs<S> p;
     p.x = x; p.old = old; p.out = out; p.veff = static_cast<const S *>(veff);
