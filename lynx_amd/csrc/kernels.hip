@@ -226,13 +226,15 @@ __global__ void __launch_bounds__(NT) k_stencil_step(StepArgs<typename Tr<S>::A>
 // of 24, and the sums are formed outside the branch of the store: inside it
 // every LDS value lived until the branch (198 registers, now 160: three waves
 // per SIMD instead of two).  90^3 x 480 float 1267 -> 1050 us a step, 60^3 x
-// 160 bfloat16 116 -> 93 us, double 236 -> 207 us.
-template <class S, int VW, int RV, int HP>
+// 160 bfloat16 116 -> 93 us, double 236 -> 207 us.  bfloat16 runs stay packed
+// until a plane is computed (unpacked at the load, every plane waited for its
+// own loads), and one run per thread is held to four waves per SIMD: 87 us.
+template <class S, class T, int VW, int RV, int HP>
 struct VecLoads {
-    VRun<S, VW> front[RV];
-    VRun<S, VW> old[RV];
+    Held<S, T, VW> front[RV];
+    Held<S, T, VW> old[RV];
     VRun<S, VW> v[RV];
-    VRun<S, VW> halo[HP];
+    Held<S, T, VW> halo[HP];
 };
 
 // lap[r] += sum_k c[k] (row y_r + k, row y_r - k) for the RV runs of a thread in
@@ -343,24 +345,24 @@ __device__ __forceinline__ void stencil_vec_body(const StepArgs<S> &p, const Ste
         hx0[h] = v ? xx : kNoX;
     }
 
-    auto load_plane = [&](int zz, VRun<S, VW> *dst) {
+    auto load_plane = [&](int zz, Held<S, T, VW> *dst) {
         if (zz < 0) zz += nz;
         else if (zz >= nz) zz -= nz;
         const T *src = X + zz * nxny;
 #pragma unroll
-        for (int r = 0; r < RV; ++r) dst[r] = vldc<VW, S>(src, qoff[r]);
+        for (int r = 0; r < RV; ++r) dst[r] = vldh<VW, S>(src, qoff[r]);
     };
-    auto issue = [&](int zs, VecLoads<S, VW, RV, HP> &L) {
+    auto issue = [&](int zs, VecLoads<S, T, VW, RV, HP> &L) {
         zs = min(zs, z1 - 1);
         load_plane(zs + R, L.front);
         const int zo = zs * nxny;
 #pragma unroll
         for (int r = 0; r < RV; ++r) {
-            L.old[r] = has_old ? vldc<VW, S>(O + zo, qoff[r]) : vzero<S, VW>();
+            if (has_old) L.old[r] = vldh<VW, S>(O + zo, qoff[r]);
             L.v[r] = vld<VW>(p.veff + zo, qoff[r]);
         }
 #pragma unroll
-        for (int h = 0; h < HP; ++h) L.halo[h] = vldc<VW, S>(X + zo, hsrc[h]);
+        for (int h = 0; h < HP; ++h) L.halo[h] = vldh<VW, S>(X + zo, hsrc[h]);
     };
     // a run, and one wrapped copy of it when it lies within XO of an x face
     // (x + nx to the right of the row, x - nx to the left; nx >= 2 XO, so a
@@ -376,24 +378,24 @@ __device__ __forceinline__ void stencil_vec_body(const StepArgs<S> &p, const Ste
     VRun<S, VW> ring[RV][NR];
 #pragma unroll
     for (int i = 0; i < 2 * R; ++i) {
-        VRun<S, VW> tmp[RV];
+        Held<S, T, VW> tmp[RV];
         load_plane(z0 - R + i, tmp);
 #pragma unroll
-        for (int r = 0; r < RV; ++r) ring[r][i] = tmp[r];
+        for (int r = 0; r < RV; ++r) ring[r][i] = tmp[r].get();
     }
 
     const S diag = p.c[0][0] + p.c[1][0] + p.c[2][0];
     int buf = 0;
-    auto step = [&](int z, VecLoads<S, VW, RV, HP> &cur, VecLoads<S, VW, RV, HP> &nxt) {
+    auto step = [&](int z, VecLoads<S, T, VW, RV, HP> &cur, VecLoads<S, T, VW, RV, HP> &nxt) {
         issue(z + 1, nxt);
         S *L = lds + buf * plane;
 #pragma unroll
         for (int r = 0; r < RV; ++r) {
-            ring[r][2 * R] = cur.front[r];
+            ring[r][2 * R] = cur.front[r].get();
             put(L, qli[r], qx0[r], ring[r][R]);
         }
 #pragma unroll
-        for (int h = 0; h < HP; ++h) put(L, hli[h], hx0[h], cur.halo[h]);
+        for (int h = 0; h < HP; ++h) put(L, hli[h], hx0[h], cur.halo[h].get());
         __syncthreads();
         T *Yz = Y + z * nxny;
         VRun<S, VW> lap[RV], own[RV];
@@ -427,11 +429,12 @@ __device__ __forceinline__ void stencil_vec_body(const StepArgs<S> &p, const Ste
 #pragma unroll
         for (int r = 0; r < RV; ++r) {
             VRun<S, VW> res;
+            const VRun<S, VW> old = cur.old[r].get();
 #pragma unroll
             for (int e = 0; e < VW; ++e) {
                 const S hval = fm(cur.v[r].v[e] + io.s, ring[r][R].v[e], S(-0.5) * lap[r].v[e]);
                 res.v[e] = io.a * hval;
-                if (has_old) res.v[e] = fm(io.b, cur.old[r].v[e], res.v[e]);
+                if (has_old) res.v[e] = fm(io.b, old.v[e], res.v[e]);
             }
             if (qv[r]) vstc<VW>(Yz, qoff[r], res);
         }
@@ -442,7 +445,7 @@ __device__ __forceinline__ void stencil_vec_body(const StepArgs<S> &p, const Ste
         buf ^= 1;
     };
 
-    VecLoads<S, VW, RV, HP> la, lb;
+    VecLoads<S, T, VW, RV, HP> la, lb;
     issue(z0, la);
     int z = z0;
     for (; z + 1 < z1; z += 2) {
@@ -453,7 +456,7 @@ __device__ __forceinline__ void stencil_vec_body(const StepArgs<S> &p, const Ste
 }
 
 template <class S, int R, int RV, int NT, int HP, int W, int VW, class T>
-__global__ void __launch_bounds__(NT) k_stencil_vec(StepArgs<S> p)
+__global__ void __launch_bounds__(NT, sizeof(T) == 2 && RV == 1 ? 4 : 1) k_stencil_vec(StepArgs<S> p)
 {
     const int w = xcd_work_item();
     if (w >= p.nwork) return;
@@ -550,24 +553,24 @@ __device__ __forceinline__ void stencil_vacc_body(const StepArgs<S> &p, const St
     auto phys = [&](int f) { return down ? z0 + z1 - 1 - f : f; };
     // loads for plane f: its owned runs (z-wrapped), and, for planes of the
     // chunk, its halo runs and Veff; Y_{k-2} of output plane f - R
-    auto issue = [&](int f, VecLoads<S, VW, RV, HP> &L) {
+    auto issue = [&](int f, VecLoads<S, T, VW, RV, HP> &L) {
         f = min(f, f_end);
         int zz = phys(f);
         if (zz < 0) zz += nz;
         else if (zz >= nz) zz -= nz;
         const T *Xz = X + zz * nxny;
 #pragma unroll
-        for (int r = 0; r < RV; ++r) L.front[r] = vldc<VW, S>(Xz, qoff[r]);
+        for (int r = 0; r < RV; ++r) L.front[r] = vldh<VW, S>(Xz, qoff[r]);
         if (f >= z0 && f < z1) {
 #pragma unroll
-            for (int h = 0; h < HP; ++h) L.halo[h] = vldc<VW, S>(Xz, hsrc[h]);
+            for (int h = 0; h < HP; ++h) L.halo[h] = vldh<VW, S>(Xz, hsrc[h]);
 #pragma unroll
             for (int r = 0; r < RV; ++r) L.v[r] = vld<VW>(p.veff + zz * nxny, qoff[r]);
         }
         if (has_old && f - R >= z0) {
             const int zo = phys(f - R) * nxny;
 #pragma unroll
-            for (int r = 0; r < RV; ++r) L.old[r] = vldc<VW, S>(O + zo, qoff[r]);
+            for (int r = 0; r < RV; ++r) L.old[r] = vldh<VW, S>(O + zo, qoff[r]);
         }
     };
     auto put = [&](S *L, int li, int x0, const VRun<S, VW> &v) {   // as in stencil_vec_body
@@ -587,14 +590,17 @@ __device__ __forceinline__ void stencil_vacc_body(const StepArgs<S> &p, const St
     const S diag = p.c[0][0] + p.c[1][0] + p.c[2][0];
     int buf = 0;
     // PD: planes of loads in flight ahead of the one consumed (1 or 2)
-    auto step = [&](int f, VecLoads<S, VW, RV, HP> &cur, VecLoads<S, VW, RV, HP> &nxt) {
+    auto step = [&](int f, VecLoads<S, T, VW, RV, HP> &cur, VecLoads<S, T, VW, RV, HP> &nxt) {
         issue(f + PD, nxt);
+        VRun<S, VW> front[RV];
+#pragma unroll
+        for (int r = 0; r < RV; ++r) front[r] = cur.front[r].get();
         if (f >= z0 && f < z1) {
             S *L = lds + buf * plane;
 #pragma unroll
-            for (int r = 0; r < RV; ++r) put(L, qli[r], qx0[r], cur.front[r]);
+            for (int r = 0; r < RV; ++r) put(L, qli[r], qx0[r], front[r]);
 #pragma unroll
-            for (int h = 0; h < HP; ++h) put(L, hli[h], hx0[h], cur.halo[h]);
+            for (int h = 0; h < HP; ++h) put(L, hli[h], hx0[h], cur.halo[h].get());
             __syncthreads();
             VRun<S, VW> lap[RV];
 #pragma unroll
@@ -608,14 +614,14 @@ __device__ __forceinline__ void stencil_vacc_body(const StepArgs<S> &p, const St
                 }
 #pragma unroll
                 for (int e = 0; e < VW; ++e)
-                    lap[r].v[e] = fm(diag - S(2) * (cur.v[r].v[e] + io.s), cur.front[r].v[e], acc[r][R].v[e]);
+                    lap[r].v[e] = fm(diag - S(2) * (cur.v[r].v[e] + io.s), front[r].v[e], acc[r][R].v[e]);
 #pragma unroll
                 for (int k = 1; k <= R; ++k)
 #pragma unroll
                     for (int e = 0; e < VW; ++e)
                         lap[r].v[e] = fm(p.c[0][k], add(xr[XO + e + k], xr[XO + e - k]), lap[r].v[e]);
                 }
-            add_rows<S, R, RV, W, VW>(L + qli[0], p.c[1], cur.front, lap);
+            add_rows<S, R, RV, W, VW>(L + qli[0], p.c[1], front, lap);
 #pragma unroll
             for (int r = 0; r < RV; ++r) acc[r][R] = lap[r];
             buf ^= 1;
@@ -628,7 +634,7 @@ __device__ __forceinline__ void stencil_vacc_body(const StepArgs<S> &p, const St
                 if (j == R) continue;
                 const int d = j < R ? R - j : j - R;
 #pragma unroll
-                for (int e = 0; e < VW; ++e) acc[r][j].v[e] = fm(p.c[2][d], cur.front[r].v[e], acc[r][j].v[e]);
+                for (int e = 0; e < VW; ++e) acc[r][j].v[e] = fm(p.c[2][d], front[r].v[e], acc[r][j].v[e]);
             }
         if (f - R >= z0) {
             const int zp = phys(f - R);
@@ -636,10 +642,11 @@ __device__ __forceinline__ void stencil_vacc_body(const StepArgs<S> &p, const St
 #pragma unroll
             for (int r = 0; r < RV; ++r) {
                 VRun<S, VW> res;
+                const VRun<S, VW> old = cur.old[r].get();
 #pragma unroll
                 for (int e = 0; e < VW; ++e) {
                     res.v[e] = (S(-0.5) * io.a) * acc[r][0].v[e];
-                    if (has_old) res.v[e] = fm(io.b, cur.old[r].v[e], res.v[e]);
+                    if (has_old) res.v[e] = fm(io.b, old.v[e], res.v[e]);
                 }
                 if (qv[r]) vstc<VW>(Yz, qoff[r], res);
             }
@@ -654,7 +661,7 @@ __device__ __forceinline__ void stencil_vacc_body(const StepArgs<S> &p, const St
 
     int f = z0 - R;
     if constexpr (PD == 1) {
-        VecLoads<S, VW, RV, HP> la, lb;
+        VecLoads<S, T, VW, RV, HP> la, lb;
         issue(f, la);
         for (; f + 1 <= f_end; f += 2) {
             step(f, la, lb);
@@ -664,7 +671,7 @@ __device__ __forceinline__ void stencil_vacc_body(const StepArgs<S> &p, const St
     } else {
         // three load sets in rotation: the set refilled at step f is the
         // one consumed at step f - 1
-        VecLoads<S, VW, RV, HP> la, lb, lc;
+        VecLoads<S, T, VW, RV, HP> la, lb, lc;
         issue(f, la);
         issue(f + 1, lb);
         for (; f + 2 <= f_end; f += 3) {

@@ -46,9 +46,7 @@ template <class T> struct StoreAs;
 template <> struct StoreAs<bf16> {
     static __device__ __forceinline__ bf16 from(float f)
     {
-        unsigned u = __float_as_uint(f);
-        u += 0x7fffu + ((u >> 16) & 1u);
-        return bf16{(unsigned short)(u >> 16)};
+        return __builtin_bit_cast(bf16, (__bf16)f);   // v_cvt_pk_bf16_f32
     }
 };
 template <> struct StoreAs<float> { static __device__ __forceinline__ float from(float f) { return f; } };
@@ -259,20 +257,32 @@ __device__ __forceinline__ VRun<S, VW> vld(const S *base, unsigned i)
     return *reinterpret_cast<const VRun<S, VW> *>(reinterpret_cast<const char *>(base) + i * (unsigned)sizeof(S));
 }
 
-// a run of storage type T loaded into compute type S, and stored back
-template <int VW, class S, class T>
-__device__ __forceinline__ VRun<S, VW> vldc(const T *base, unsigned i)
-{
-    if constexpr (std::is_same<S, T>::value) {
-        return vld<VW>(base, i);
-    } else {
-        const VRun<T, VW> t = vld<VW>(base, i);
-        VRun<S, VW> r;
+// A run of storage type T as it was loaded, and its values in compute type S.
+// bfloat16 pairs stay packed until they are used: unpacked at the load, the
+// values would wait for memory where the loads are issued, a plane too early.
+template <class S, class T, int VW>
+struct Held {
+    VRun<S, VW> r;
+    __device__ __forceinline__ VRun<S, VW> get() const { return r; }
+};
+template <int VW>
+struct alignas(2 * VW) Held<float, bf16, VW> {
+    unsigned w[VW / 2];
+    __device__ __forceinline__ VRun<float, VW> get() const
+    {
+        VRun<float, VW> r;
 #pragma unroll
-        for (int e = 0; e < VW; ++e) r.v[e] = to_compute(t.v[e]);
+        for (int e = 0; e < VW; ++e)
+            r.v[e] = __uint_as_float(e & 1 ? w[e / 2] & 0xffff0000u : w[e / 2] << 16);
         return r;
     }
+};
+template <int VW, class S, class T>
+__device__ __forceinline__ Held<S, T, VW> vldh(const T *base, unsigned i)
+{
+    return *reinterpret_cast<const Held<S, T, VW> *>(reinterpret_cast<const char *>(base) + i * (unsigned)sizeof(T));
 }
+// a run stored back as T
 template <int VW, class S, class T>
 __device__ __forceinline__ void vstc(T *base, unsigned i, const VRun<S, VW> &v)
 {
