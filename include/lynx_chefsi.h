@@ -359,7 +359,8 @@ lynx_status lynx_get_grid_dims(const lynx_ctx *ctx, int dims[3]);
  * on output), the timed candidates in order vector_runs 0..3 x row alignment
  * 0..1 (none for 0) x threads
  * 256..512 x points_div 1..2 x z_chunks 1..4 (shapes that do not fit a grid
- * are skipped). */
+ * are skipped; blocks too small to fill the chip have chunks of down to three
+ * planes beside or instead of these). */
 lynx_status lynx_set_stencil_config(lynx_ctx *ctx, int threads, int points_div, int z_chunks,
                                     int vector_runs);
 lynx_status lynx_get_stencil_config(const lynx_ctx *ctx, int dtype, int ncol, int *threads,

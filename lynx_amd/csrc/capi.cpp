@@ -297,14 +297,30 @@ void upload_phases(lynx_ctx *c)
 // timed on the caller's own data (plain H application into the destination
 // block, which the real step overwrites afterwards); the fastest is cached
 // for this grid shape, element type and column count.
-std::vector<gpu::StepCfg> step_candidates(const lynx_ctx *c, int e)
+//
+// A launch has about nx ny ncol lanes per z chunk and the chip holds 256 CUs x
+// 1024 of them.  Where four chunks leave it mostly idle the march along z is
+// what takes the time, and chunks down to three planes (each reads 2R more)
+// are timed too; orthogonal launches with lanes for an eighth of the chip or
+// less have those only, so that the first call stays as short.  Filters of
+// degree 20 and an apply, double: 30^3 x 24 434 -> 297 us, 20^3 x 12 31.8 ->
+// 24 us; at 47 x 45 x 51 x 61 and complex 40^3 x 48 (half and 0.3 of the chip)
+// more than three chunks are slower.
+std::vector<gpu::StepCfg> step_candidates(const lynx_ctx *c, int e, int ncol)
 {
     std::vector<gpu::StepCfg> v;
+    const int fill = (int)(256L * 1024 / std::max(1L, (long)c->st.nx * c->st.ny * ncol));
+    const int fine = std::min(fill, (c->st.nz + 2) / 3);
+    std::vector<int> chunks;
+    if (fill < 8 || fine <= 4 || !c->lat.orth)
+        for (int nz : {1, 2, 3, 4})
+            if (nz == 1 || c->st.nz / nz >= 2 * gpu::kMaxR) chunks.push_back(nz);
+    if (fine > 4) chunks.push_back(fine);
     for (int vec : {0, 1, 2, 3})
       for (int align : {0, 1})
         for (int nt : {256, 512})
             for (int div : {1, 2})
-                for (int nz : {1, 2, 3, 4}) {
+                for (int nz : chunks) {
                     if (align && !vec) continue;
                     gpu::StepCfg k;
                     k.rp_div = div;
@@ -312,7 +328,6 @@ std::vector<gpu::StepCfg> step_candidates(const lynx_ctx *c, int e)
                     k.nt = nt;
                     k.vec = vec;
                     k.align = align;
-                    if (nz > 1 && c->st.nz / nz < 2 * gpu::kMaxR) continue;
                     if (vec && !c->lat.orth) continue;   // the non-orthogonal kernel has one form
                     if (!gpu::stencil_shape_fits(e, c->st.nx, k)) continue;
                     v.push_back(k);
@@ -328,7 +343,7 @@ const gpu::StepCfg &step_config(lynx_ctx *c, int e, const void *x, long ldx, voi
     if (it != c->tuned.end()) return it->second;
     gpu::StepCfg best{};
     if (c->autotune) {
-        const auto cands = step_candidates(c, e);
+        const auto cands = step_candidates(c, e, ncol);
         hipEvent_t e0, e1;
         HIP_OK(hipEventCreate(&e0));
         HIP_OK(hipEventCreate(&e1));
@@ -374,7 +389,7 @@ const gpu::StepCfg &step_config(lynx_ctx *c, int e, const void *x, long ldx, voi
     }
     if (!gpu::stencil_shape_fits(e, c->st.nx, best)) {
         // untuned: the first shape that fits the rows (long rows need 512 threads)
-        const auto cands = step_candidates(c, e);
+        const auto cands = step_candidates(c, e, ncol);
         if (!cands.empty()) best = cands.front();
     }
     return c->tuned[key] = best;
@@ -386,7 +401,7 @@ const gpu::StepCfg &step_config(lynx_ctx *c, int e, const void *x, long ldx, voi
 bool bf16_filter_fits(const lynx_ctx *c)
 {
     if (!c->lat.orth) return false;
-    for (const auto &k : step_candidates(c, gpu::B16))
+    for (const auto &k : step_candidates(c, gpu::B16, 1))
         if (k.vec) return true;
     return false;
 }

@@ -50,7 +50,7 @@ def test_points_step_matches_oracle(n, skew):
         H.set_kpoint(k)
         X = s.random_block(3, 41, cplx).astype(dt)
         ref = op.apply(X.astype(complex if cplx else float), s.veff, c=-0.2)
-        for shape in [(t, d, z) for t in (256, 512) for d in (1, 2) for z in (1, 2)]:
+        for shape in [(t, d, z) for t in (256, 512) for d in (1, 2) for z in (1, 2, (n[2] + 2) // 3)]:
             L.check(L.lib().lynx_set_stencil_config(H.ctx, *shape, 0), H.ctx)
             got = H._apply(X.T.copy(), s.veff, -0.2, dt).reshape(3, -1).T
             assert rel(got, ref) < (2e-6 if single else 1e-12), (dt, shape)

@@ -2,7 +2,8 @@
 share their LDS reads) at the edges of the bands, against the oracle: an odd
 number of rows (the last thread row owns one run and needs the row beyond the
 band, wrapped or not), one row, fewer rows than threads, several bands, runs
-of two and of four points, both directions of a z-chunk.  Bars of the other
+of two and of four points, both directions of a
+z-chunk, chunks of three planes.  Bars of the other
 stencil tests: 1e-12 (FP64) and 2e-6 (single precision) per apply, 1e-11 and
 2e-5 per filter."""
 import numpy as np
@@ -32,7 +33,7 @@ def test_run_vector_rows_match_oracle(n):
         X = s.random_block(3, 43, False).astype(dt)
         one = op.apply(X.astype(float), s.veff, c=-0.2)
         five = op.cheb_filter(X.astype(float), s.veff, lc, lo, hi, 5)
-        for shape in [(t, d, z, v) for t in (256, 512) for d in (1, 2) for z in (1, 2) for v in (1, 2, 3, 5, 6, 7)]:
+        for shape in [(t, d, z, v) for t in (256, 512) for d in (1, 2) for z in (1, 2, (n[2] + 2) // 3) for v in (1, 2, 3, 5, 6, 7)]:
             L.check(L.lib().lynx_set_stencil_config(H.ctx, *shape), H.ctx)
             got = H._apply(X.T.copy(), s.veff, -0.2, dt).reshape(3, -1).T
             assert rel(got, one) < (2e-6 if single else 1e-12), (dt, shape)
