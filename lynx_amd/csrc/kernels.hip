@@ -1061,7 +1061,8 @@ __global__ void __launch_bounds__(256) k_lanczos_update(S *y, S *x, S *z, double
     double s = 0.0;
     for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
         // y -= a*x + b*z  (evaluated as in Lanczos.hpp:162-165)
-        S t = add(scl((A)a, x[i]), scl((A)b, z[i]));
+        // the first update has no z yet: whatever its memory holds (0 * NaN) stays out
+        S t = add(scl((A)a, x[i]), b != 0.0 ? scl((A)b, z[i]) : zero<S>());
         S v = add(y[i], scl(A(-1), t));
         y[i] = v;
         z[i] = x[i];
