@@ -580,7 +580,8 @@ lynx_status lynx_batch_last_timing(const lynx_batch *batch, double *ms, int *lau
  * filter; H times the orthonormalised blocks is one batched step; the
  * Gram products and rotations are batched GEMMs and the Cholesky
  * factorisations, triangular inverses and subspace eigensolves batched
- * rocSOLVER calls, over the units of equal (Nd, ncol, ldpsi).  dtype is
+ * rocSOLVER calls (up to 64 real or 32 complex columns: kernels of the
+ * library's own), over the units of equal (Nd, ncol, ldpsi).  dtype is
  * LYNX_F64 or LYNX_C128.  eigvals receives sum(ncol) values, unit after
  * unit, ascending within a unit; lambda_cutoff_out[u] (optional) the
  * unit's eig[ncol - 1] + 0.1.  Replaces the per-(spin, k-point) loop of

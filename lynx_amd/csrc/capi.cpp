@@ -652,7 +652,7 @@ void gram(lynx_ctx *c, int e, const void *A, long lda, const void *B, long ldb, 
         gpu::gram_f64_fits(static_cast<const double *>(A), lda, static_cast<const double *>(B), ldb)) {
         // a symmetric result (the overlap A^T A, or the projection whose
         // Hermitian part is taken): the hand-written FP64 MFMA kernel forms
-        // only the upper tiles (5.8 against 7.5 ms for rocBLAS's full
+        // only the upper tiles (3.4 against 7.5 ms for rocBLAS's full
         // product at 729,000 x 480); general products stay rocBLAS GEMMs,
         // which run them faster than this kernel
         const int ns = gpu::gram_f64_splits(nd, n);
