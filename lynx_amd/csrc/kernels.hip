@@ -6,6 +6,7 @@
 #include "kernels_nonlocal.hpp"
 #include "kernels_points.hpp"
 #include "stencil_common.hpp"
+#include "stencil_lanes.hpp"
 
 #include <hip/hip_runtime.h>
 #include <algorithm>
@@ -56,7 +57,7 @@ __device__ __forceinline__ void stencil_step_body(const StepArgs<typename Tr<S>:
     // the writes of idle lanes and of elements without a ghost copy (no
     // branches, and no two lanes of a wave writing the same address)
     const int dummy = W * (p.tyr + 2 * R) + (int)threadIdx.x;
-    const int plane = W * (p.tyr + 2 * R) + NT;
+    const int plane = plane_elems(W, R, p.tyr, NT, 1);
 
     const int band = w % p.nbands;
     const int rest = w / p.nbands;
@@ -75,8 +76,9 @@ __device__ __forceinline__ void stencil_step_body(const StepArgs<typename Tr<S>:
 
     const int tid = threadIdx.x;
     const int npts = rows * nx;
-    // owned points: plane offset (0 for idle lanes), LDS index and the LDS
-    // indices of its wrapped x-ghost copies (dummy when none)
+    // owned points: plane offset, LDS index and the LDS indices of its wrapped
+    // x-ghost copies (dummy when none); slots beyond the band repeat its
+    // points, all but the store of the result
     unsigned qoff[RP];   // element offsets within a plane
     int qli[RP], qgh[RP], qgl[RP];
     bool qv[RP];
@@ -84,14 +86,13 @@ __device__ __forceinline__ void stencil_step_body(const StepArgs<typename Tr<S>:
     for (int r = 0; r < RP; ++r) {
         const int q = tid + r * NT;
         qv[r] = q < npts;
-        const int qq = qv[r] ? q : 0;
+        const int qq = band_point(q, npts);
         const int qy = qq / nx;
         const int qx = qq - qy * nx;
-        qoff[r] = qv[r] ? (y0 + qy) * nx + qx : 0;
-        const int li = (qy + R) * W + qx + R;
-        qli[r] = qv[r] ? li : dummy;
-        qgh[r] = (qv[r] && qx < R) ? li + nx : dummy;
-        qgl[r] = (qv[r] && qx >= nx - R) ? li - nx : dummy;
+        qoff[r] = (y0 + qy) * nx + qx;
+        qli[r] = plane_at(W, R, R, qy, qx);
+        qgh[r] = qx < R ? qli[r] + nx : dummy;
+        qgl[r] = qx >= nx - R ? qli[r] - nx : dummy;
     }
     // halo slots: R rows below and R above the band, wrapped in y
     const int nh = 2 * R * nx;
@@ -281,7 +282,7 @@ __device__ __forceinline__ void stencil_vec_body(const StepArgs<S> &p, const Ste
 
     const int nx = p.nx, ny = p.ny, nz = p.nz;
     const int base = W * (p.tyr + 2 * R);
-    const int plane = base + NT * VW;            // + one dummy run per lane
+    const int plane = plane_elems(W, R, p.tyr, NT, VW);
 
     const int band = w % p.nbands;
     const int rest = w / p.nbands;
@@ -300,10 +301,10 @@ __device__ __forceinline__ void stencil_vec_body(const StepArgs<S> &p, const Ste
 
     const int tid = threadIdx.x;
     const int dummy = base + tid * VW;
-    // owned runs: plane offset (element index), LDS index and x of the first
-    // element (kNoX for lanes without a run, whose stores go to the dummy).
-    // Lane q takes run q % lpr of the RV band rows from RV (q / lpr) on, which
-    // share their y neighbours' LDS reads; with lpr a multiple of 16
+    // the lane's runs (run_lane; the adjacent rows share their y neighbours'
+    // LDS reads): plane offset (element index), LDS index and x of the first
+    // element (kNoX: a halo slot without a run, which writes to the dummy).
+    // With lpr a multiple of 16
     // no group of 16 lanes (one LDS cycle of 16-byte accesses) straddles two
     // rows, so row starts never collide in the same banks.
     constexpr int kNoX = -(1 << 20);
@@ -314,17 +315,11 @@ __device__ __forceinline__ void stencil_vec_body(const StepArgs<S> &p, const Ste
     bool qv[RV];
 #pragma unroll
     for (int r = 0; r < RV; ++r) {
-        const int q0 = tid / lpr;
-        const int qr = tid - q0 * lpr;
-        const int qy = RV * q0 + r;
-        qv[r] = qy < rows && qr < runs;
-        const int qx = qv[r] ? qr * VW : 0;
-        const int qyy = qv[r] ? qy : 0;
-        qoff[r] = qv[r] ? (y0 + qyy) * nx + qx : 0;
-        // a row above an odd band: the loaded run is the neighbour of run 0
-        if (r > 0 && !qv[r] && qv[0]) qoff[r] = (y0 + qy < ny ? y0 + qy : 0) * nx + qx0[0];
-        qli[r] = qv[r] ? (qyy + R) * W + XO + qx : dummy;
-        qx0[r] = qv[r] ? qx : kNoX;
+        const RunLane q = run_lane(tid, r, RV, lpr, runs, rows, VW);
+        qv[r] = q.own;
+        qoff[r] = (y0 + q.y < ny ? y0 + q.y : 0) * nx + q.x;
+        qli[r] = plane_at(W, R, XO, q.y, q.x);
+        qx0[r] = q.x;
     }
     unsigned hsrc[HP];
     int hli[HP], hx0[HP];
@@ -483,7 +478,7 @@ __device__ __forceinline__ void stencil_vacc_body(const StepArgs<S> &p, const St
 
     const int nx = p.nx, ny = p.ny, nz = p.nz;
     const int base = W * (p.tyr + 2 * R);
-    const int plane = base + NT * VW;
+    const int plane = plane_elems(W, R, p.tyr, NT, VW);
 
     const int band = w % p.nbands;
     const int rest = w / p.nbands;
@@ -511,17 +506,11 @@ __device__ __forceinline__ void stencil_vacc_body(const StepArgs<S> &p, const St
     bool qv[RV];
 #pragma unroll
     for (int r = 0; r < RV; ++r) {
-        const int q0 = tid / lpr;
-        const int qr = tid - q0 * lpr;
-        const int qy = RV * q0 + r;
-        qv[r] = qy < rows && qr < runs;
-        const int qx = qv[r] ? qr * VW : 0;
-        const int qyy = qv[r] ? qy : 0;
-        qoff[r] = qv[r] ? (y0 + qyy) * nx + qx : 0;
-        // a row above an odd band: the loaded run is the neighbour of run 0
-        if (r > 0 && !qv[r] && qv[0]) qoff[r] = (y0 + qy < ny ? y0 + qy : 0) * nx + qx0[0];
-        qli[r] = qv[r] ? (qyy + R) * W + XO + qx : dummy;
-        qx0[r] = qv[r] ? qx : kNoX;
+        const RunLane q = run_lane(tid, r, RV, lpr, runs, rows, VW);
+        qv[r] = q.own;
+        qoff[r] = (y0 + q.y < ny ? y0 + q.y : 0) * nx + q.x;
+        qli[r] = plane_at(W, R, XO, q.y, q.x);
+        qx0[r] = q.x;
     }
     unsigned hsrc[HP];
     int hli[HP], hx0[HP];
@@ -1220,7 +1209,7 @@ void launch_step_rp(const StencilGeom &g, const void *x, long ldx, const void *o
         for (int sd = 0; sd < 2; ++sd)
             for (int q = 0; q < 2; ++q) p.ph[ax][sd][q] = (A)g.phase[ax][sd][q];
     const int blocks = ((p.nwork + 7) / 8) * 8;
-    const size_t shm = 2 * sizeof(S) * ((size_t)pitch * (p.tyr + 2 * kMaxR) + NT);
+    const size_t shm = 2 * sizeof(S) * (size_t)plane_elems(pitch, kMaxR, p.tyr, NT, 1);
     hipLaunchKernelGGL((k_stencil_step<S, kMaxR, RP, NT, kLongHalo, 256>), dim3(blocks), dim3(NT), shm, st, p);
 }
 
@@ -1273,7 +1262,7 @@ bool launch_step_vec(const StencilGeom &g, const void *x, long ldx, const void *
             for (int q = 0; q < 2; ++q) p.ph[ax][sd][q] = (S)g.phase[ax][sd][q];
     const int blocks = ((p.nwork + 7) / 8) * 8;
     const int pitch = g.nx + 2 * XO <= 64 ? 64 : 128;
-    const size_t shm = 2 * sizeof(S) * ((size_t)pitch * (p.tyr + 2 * kMaxR) + NT * VW);
+    const size_t shm = 2 * sizeof(S) * (size_t)plane_elems(pitch, kMaxR, p.tyr, NT, VW);
     const bool small_halo = 2 * kMaxR * lpr <= NT * HS;
     auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(blocks), dim3(NT), shm, st, p); };
     if constexpr (MODE > 0) {
@@ -1809,7 +1798,7 @@ void batch_step(BatchPlan *P, int step, int ix, int iold, int iout, bool first, 
                 continue;
             }
             if constexpr (!Tr<S>::C) {
-                const size_t shm = 2 * sizeof(S) * (256 * (size_t)(G.max_tyr + 2 * kMaxR) + 512);
+                const size_t shm = 2 * sizeof(S) * (size_t)plane_elems(256, kMaxR, G.max_tyr, 512, 1);
                 hipLaunchKernelGGL((k_stencil_batch<S, batch_rp_orth<S>()>), dim3((G.nitems + 7) / 8 * 8), dim3(512),
                                    shm, st, static_cast<const BatchRec<S> *>(P->recs), G.items, G.nitems,
                                    static_cast<const S *>(cf), ix, iold, iout);
