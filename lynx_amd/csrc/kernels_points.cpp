@@ -12,6 +12,25 @@ namespace {
 constexpr long kLds = 160 * 1024;   // LDS of a workgroup (gfx950)
 
 int round64(int n) { return (n + 63) / 64 * 64; }
+
+// complex128 kernels with six halo points per thread hold more than a thread's
+// registers, but for the orthogonal one that marches beyond the z boundary
+bool spills(int e, bool orth, const PointShape &s) { return e == C128 && s.hp == 6 && (!orth || s.wrapz); }
+
+// Whether a march that wraps in z (nz planes instead of nz + 2R) is worth the
+// LDS of its end planes' parts: the workgroups left on a CU must hide each
+// other's latency.  Without / with it, us for six steps of a batch by waves
+// per CU: double 60^3 x 108 orthogonal 8 waves 1337 / 1423, 9 waves 1483 /
+// 1413, 40^3 x 370 12 waves 1333 / 1220; complex64 72^3 8 waves 807 / 904;
+// complex128 40^3 4 waves 1115 / 1345, skew 60^3 4 waves 1648 / 1949 and 48^3
+// 6 waves 1825 / 1537; double skew 8 waves 1833 / 1876 (256 threads), 2259 /
+// 2069 (512).
+bool wrap_pays(int e, bool orth, PointShape s, long lds)
+{
+    s.wrapz = true;
+    const int waves = (int)(kLds / lds) * (s.nt / 64);
+    return waves > (orth && e != C128 ? 8 : 4) && !spills(e, orth, s);
+}
 }  // namespace
 
 bool point_shape(int e, const StencilGeom &g, int max_threads, int nzch, PointShape &out)
@@ -35,7 +54,7 @@ bool point_shape(int e, const StencilGeom &g, int max_threads, int nzch, PointSh
             if (2 * R * nx <= hs[k] * s.nt) s.hp = hs[k];
         const long planes = 2 * es * s.pitch * ((s.tyr + 2 * R) + (g.orth ? 0 : s.tyr));
         const long stash = 2 * R * es * s.nt;
-        s.wrapz = s.nzch == 1 && g.nz >= 2 * R && planes + stash <= kLds;
+        s.wrapz = s.nzch == 1 && g.nz >= 2 * R && planes + stash <= kLds && wrap_pays(e, g.orth, s, planes + stash);
         s.lds = (size_t)(planes + (s.wrapz ? stash : 0));
         if (planes > kLds) continue;
         out = s;
@@ -58,6 +77,7 @@ bool point_shape_batch(int e, const StencilGeom &g, PointShape &out)
     for (int budget : {128, 192, 256, 512}) {
         PointShape s;
         if (!point_shape(e, g, budget, 1, s)) continue;
+        if (spills(e, g.orth, s) && budget < 512) continue;
         const int nb = (g.ny + s.tyr - 1) / s.tyr;
         double cost = (double)nb * s.nt / ((double)g.nx * g.ny) * (1.0 + 0.12 * 2 * kMaxR / s.tyr);
         if (s.nt > 256) cost *= 1.64;

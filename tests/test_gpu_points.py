@@ -66,3 +66,29 @@ def test_points_step_matches_oracle(n, skew):
         L.check(L.lib().lynx_cheb_filter(H.ctx, L.dtype_code(dt), L.vptr(Xf), s.nd, L.vptr(Y), s.nd, 3, 5, lc, lo, hi,
                                          L.MEM_HOST), H.ctx)
         assert rel(Y, ref) < (2e-5 if single else 1e-11), dt
+
+
+@pytest.mark.parametrize("n", [(60, 9, 14), (40, 18, 12), (72, 11, 13), (116, 6, 13)])
+@pytest.mark.parametrize("skew", [False, True])
+def test_batch_shapes_match_oracle(n, skew):
+    # rows whose LDS leaves few waves on a CU: marches beyond the z boundary
+    # instead of around it, and complex128 rows of more than three halo points
+    # per thread in fewer threads
+    from lynx_amd import core
+    s = system(n, skew)
+    op, H = s.oracle_op(), s.hamiltonian()
+    H.set_veff(s.veff)
+    lo, hi = s.veff.min() - 0.5, 80.0
+    lc = lo + 0.3 * (hi - lo)
+    for dt in DTYPES:
+        cplx = np.dtype(dt).kind == "c"
+        single = np.dtype(dt).itemsize == (8 if cplx else 4)
+        k = s.kpt if cplx else (0.0, 0.0, 0.0)
+        op.set_kpoint(k)
+        X = s.random_block(3, 43, cplx).astype(dt)
+        ref = op.cheb_filter(X.astype(complex if cplx else float), s.veff, lc, lo, hi, 4)
+        bf = core.BatchFilter([(H, k), (H, k)])
+        got = bf.filter([X, X[:, :1]], 4, lc, lo, hi, dtype=dt)
+        assert rel(got[0], ref) < (2e-5 if single else 1e-11), dt
+        assert rel(got[1], ref[:, :1]) < (2e-5 if single else 1e-11), dt
+        bf.close()
