@@ -38,10 +38,18 @@ bool point_shape(int e, const StencilGeom &g, int max_threads, int nzch, PointSh
     const int R = kMaxR, nx = g.nx, ny = g.ny;
     const long es = (long)elem_size(e);
     PointShape s;
-    s.pitch = nx + 2 * R <= 40 ? 40 : (nx + 2 * R <= 64 ? 64 : (nx + 2 * R <= 128 ? 128 : 256));
-    // halo points per thread that each pitch's kernels are built for
-    const int slots[4][3] = {{1, 2, 2}, {2, 3, 3}, {2, 3, 6}, {6, 6, 6}};
-    const int *hs = slots[s.pitch == 40 ? 0 : (s.pitch == 64 ? 1 : (s.pitch == 128 ? 2 : 3))];
+    // pitches, and the halo points per thread that each one's kernels are
+    // built for.  76 is for rows of 53 to 64 points, which a pitch of 128 left
+    // with two workgroups of double on a CU instead of three: batches of
+    // 64^3 x 91 double 1384 -> 1181 us for six steps, 60^3 x 320 3321 -> 3093 us,
+    // complex64 skew 60^3 x 160 2597 -> 2205 us; alone 59^3 x 174 double 6439 ->
+    // 5743 us for 20
+    constexpr int pitches[5] = {40, 64, 76, 128, 256};
+    constexpr int slots[5][3] = {{1, 2, 2}, {2, 3, 3}, {2, 3, 3}, {2, 3, 6}, {6, 6, 6}};
+    int ip = 0;
+    while (ip < 4 && nx + 2 * R > pitches[ip]) ++ip;
+    s.pitch = pitches[ip];
+    const int *hs = slots[ip];
     if (nx + 2 * R > 256 || nx > max_threads) return false;
     s.nzch = std::max(1, std::min(nzch, g.nz));
     for (int most = std::min(ny, max_threads / nx); most >= 1; --most) {

@@ -349,6 +349,7 @@ void by_point_shape(const PointShape &s, bool nonorth, F &&f)
         switch (s.pitch) {
             case 40: halo(std::integral_constant<int, 40>{}, I1{}, I2{}, I2{}); break;
             case 64: halo(std::integral_constant<int, 64>{}, I2{}, I3{}, I3{}); break;
+            case 76: halo(std::integral_constant<int, 76>{}, I2{}, I3{}, I3{}); break;
             case 128: halo(std::integral_constant<int, 128>{}, I2{}, I3{}, I6{}); break;
             default: f(no, wz, I6{}, std::integral_constant<int, 256>{}); break;
         }

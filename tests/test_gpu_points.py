@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 SI2 = np.array([[0.05, 0.1, 0.2], [0.5, 0.55, 0.45]])
 DTYPES = [np.float64, np.complex128, np.float32, np.complex64]
 GRIDS = [(6, 6, 6), (7, 9, 11), (11, 8, 12), (12, 6, 13), (28, 7, 9), (29, 13, 8), (52, 6, 14), (53, 9, 7),
-         (116, 7, 12), (23, 37, 13)]
+         (64, 6, 13), (65, 9, 7), (116, 7, 12), (23, 37, 13)]
 
 
 def rel(a, b):
