@@ -703,8 +703,15 @@ int gram_f64_splits(long K, int N)
     const int pairs = tiles * (tiles + 1) / 2;
     // one round of the three workgroups that a CU holds: 780 items in 768
     // slots took 4.4 ms, 765 take 3.4 ms (480 columns of 90^3 points)
-    const long want = std::max(1L, 768L / pairs);
-    return (int)std::max(1L, std::min(want, (K + kDKB - 1) / kDKB));
+    constexpr long kSlots = 768;
+    const long most = (K + kDKB - 1) / kDKB;
+    long best = std::max(1L, std::min(kSlots / pairs, most));
+    // wide blocks, whose tiles alone half fill the last round, are split as
+    // far as that fills it, the partial products within a quarter of a block
+    auto fill = [&](long s) { return (double)(pairs * s) / (double)((pairs * s + kSlots - 1) / kSlots * kSlots); };
+    for (long s = best + 1; s <= std::min({8L, most, K / (4L * N)}); ++s)
+        if (fill(s) > 1.05 * fill(best)) best = s;
+    return (int)best;
 }
 
 bool gram_f64_fits(const double *A, long lda, const double *B, long ldb)

@@ -115,6 +115,24 @@ def test_fp64_gram_matches_numpy(grid, n):
     assert np.abs(c.T - ref).max() / np.abs(ref).max() < 1e-13
 
 
+def test_fp64_gram_of_a_wide_block_in_several_splits():
+    # 29 tile columns: 435 upper tiles half fill a round of the chip, so the
+    # rows are split in three (as many partials as a quarter of the block holds)
+    from lynx_amd import _lib as L
+    from lynx_amd.hipmem import DeviceArray
+    s = System((32, 32, 32), 10.0, np.zeros((0, 3)), with_nonlocal=False)
+    H = s.hamiltonian(0)
+    n = 2700
+    A = np.random.default_rng(8).uniform(-0.5, 0.5, (n, s.nd))
+    dA = DeviceArray.from_numpy(A)
+    c = np.zeros((n, n))
+    L.check(L.lib().lynx_gram(H.ctx, L.F64, dA.value, s.nd, dA.value, s.nd, n, L.dptr(c), L.MEM_DEVICE), H.ctx)
+    dA.free()
+    ref = abs(np.linalg.det(s.latvec)) / s.nd * (A @ A.T)
+    assert np.abs(c - ref).max() / np.abs(ref).max() < 1e-13
+    assert np.array_equal(c, c.T)
+
+
 def test_gram_precision_rejects_unknown_mode():
     from lynx_amd import _lib as L
     _, H = _ctx(16)
