@@ -687,15 +687,18 @@ __global__ void __launch_bounds__(NT) k_stencil_vacc(StepArgs<S> p)
 // waves take interleaved runs of the atom's sphere points (all images); each
 // lane accumulates npm projections, then a wave reduction, and the four wave
 // sums are added in a fixed order through LDS (deterministic, no atomics).
+// The body is a function of its own: written into the kernel, its last
+// coefficient load waits for the point's value, and the lanes' writes of the
+// wave sums become a tree of 24 branches (150 atoms x 40 columns of 80^3
+// float, 32 projectors: 465 us instead of 307 us).
 template <class S, int NPM, class T>
-__global__ void __launch_bounds__(256) k_nl_gather(NlArgs<typename Tr<S>::A> p, const T *__restrict__ X,
-                                                   long ldx, S *__restrict__ beta, int ncol)
+__device__ __forceinline__ void nl_gather_body(const NlArgs<typename Tr<S>::A> &p, const T *__restrict__ X,
+                                               long ldx, S *__restrict__ beta, int ncol, int at, int n)
 {
     using A = typename Tr<S>::A;
     __shared__ S part[4][NPM];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    const int at = blockIdx.x, n = blockIdx.y;
     if (n >= ncol) return;
     const int pb = p.atom_pt_off[at], pe = p.atom_pt_off[at + 1];
     const T *Xn = X + (long)n * ldx;
@@ -736,6 +739,13 @@ __global__ void __launch_bounds__(256) k_nl_gather(NlArgs<typename Tr<S>::A> p, 
         S *bn = beta + (long)n * p.n_atom * NPM + (long)at * NPM;
         bn[lane] = scl(p.gamma[at * NPM + lane], t);
     }
+}
+
+template <class S, int NPM, class T>
+__global__ void __launch_bounds__(256) k_nl_gather(NlArgs<typename Tr<S>::A> p, const T *__restrict__ X,
+                                                   long ldx, S *__restrict__ beta, int ncol)
+{
+    nl_gather_body<S, NPM, T>(p, X, ldx, beta, ncol, blockIdx.x, blockIdx.y);
 }
 
 // -------------------------------------------------------- nonlocal scatter --
