@@ -89,7 +89,8 @@ def test_split_bf16x3_gram_exact_on_bfloat16_inputs_and_device_memory():
     dA.free(); dB.free()
 
 
-@pytest.mark.parametrize("grid,n", [(16, 24), ((20, 21, 22), 300), ((24, 25, 26), 129)])
+@pytest.mark.parametrize("grid,n", [(16, 24), ((20, 21, 22), 300), ((24, 25, 26), 129), ((20, 20, 20), 65),
+                                    ((6, 7, 6), 65), ((30, 30, 29), 97)])
 def test_fp64_gram_matches_numpy(grid, n):
     from lynx_amd import _lib as L
     from lynx_amd.hipmem import DeviceArray, synchronize
