@@ -174,7 +174,8 @@ void narrow_rotate(int e, const NarrowBlocks &A, long lda, const NarrowBlocks &C
 // order of the first pivot that is not positive, or 0.
 void narrow_cholesky_inverse(int e, void *S, int n, int units, int *info, hipStream_t st);
 // H -> its eigenvectors, ascending eigenvalues in eval; info per unit: 1 when
-// the iteration did not converge.
+// the iteration did not converge or H holds a value that is not finite (H and
+// eval are then unchanged).
 void narrow_eig(int e, void *H, int n, int units, double *eval, int *info, hipStream_t st);
 // Small dense helpers on n x n column-major matrices.
 void hermitian_part(int e, void *H, int n, hipStream_t st);

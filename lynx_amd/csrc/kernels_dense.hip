@@ -251,6 +251,13 @@ __device__ __forceinline__ double real_(double a) { return a; }
 __device__ __forceinline__ double real_(Cx a) { return a.re; }
 __device__ __forceinline__ double abs_(double a) { return fabs(a); }
 __device__ __forceinline__ double abs_(Cx a) { return hypot(a.re, a.im); }
+__device__ __forceinline__ double peak(double a) { return fabs(a); }           // largest component, NaN of a NaN
+__device__ __forceinline__ double peak(Cx a)
+{
+    return isnan(a.re) || isnan(a.im) ? a.re + a.im : fmax(fabs(a.re), fabs(a.im));
+}
+__device__ __forceinline__ double scale2(double a, int e) { return ldexp(a, e); }
+__device__ __forceinline__ Cx scale2(Cx a, int e) { return {ldexp(a.re, e), ldexp(a.im, e)}; }
 __device__ __forceinline__ double norm2(double a) { return a * a; }
 __device__ __forceinline__ double norm2(Cx a) { return fma(a.re, a.re, a.im * a.im); }
 template <class E> __device__ __forceinline__ E from_real(double a);
@@ -346,11 +353,42 @@ __global__ void __launch_bounds__(NT) k_narrow_eig(double *__restrict__ M, int n
         s += norm2(v);
     }
     __shared__ double red[NT / 64];
-    for (int o = 32; o; o >>= 1) s += __shfl_xor(s, o);
-    if ((t & 63) == 0) red[t >> 6] = s;
-    __syncthreads();
-    s = 0.0;
-    for (int i = 0; i < NT / 64; ++i) s += red[i];
+    auto over_threads = [&](double v, auto op) {               // over the workgroup, all threads get it
+        for (int o = 32; o; o >>= 1) v = op(v, __shfl_xor(v, o));
+        __syncthreads();
+        if ((t & 63) == 0) red[t >> 6] = v;
+        __syncthreads();
+        v = red[0];
+        for (int i = 1; i < NT / 64; ++i) v = op(v, red[i]);
+        return v;
+    };
+    auto plus = [](double a, double b) { return a + b; };
+    s = over_threads(s, plus);
+    // Squares out of range: the matrix is scaled by a power of two, or, with a
+    // value that is no number or infinite, refused (a NaN would pass every
+    // test below as converged)
+    int e = 0;
+    if (!(s <= 0x1p900) || s < 0x1p-900) {
+        double a = 0.0;
+        for (int i = t; i < m * m; i += NT) {
+            const double v = peak(A[i % m + i / m * P]);
+            a = v <= 0x1.fffffffffffffp1023 ? fmax(a, v) : HUGE_VAL;
+            if (a == HUGE_VAL) break;
+        }
+        a = over_threads(a, [](double x, double y) { return fmax(x, y); });
+        if (a == HUGE_VAL) {
+            if (t == 0) info[u] = 1;
+            return;
+        }
+        e = a > 0.0 ? ilogb(a) : 0;
+        s = 0.0;
+        for (int i = t; i < m * m; i += NT) {
+            E &v = A[i % m + i / m * P];
+            v = scale2(v, -e);
+            s += norm2(v);
+        }
+        s = over_threads(s, plus);
+    }
     const double tol = sqrt(s) * 0x1p-53;
     double big = 0.0;
     bool done = false;
@@ -444,7 +482,7 @@ __global__ void __launch_bounds__(NT) k_narrow_eig(double *__restrict__ M, int n
         int rank = 0;
         for (int j = 0; j < n; ++j) rank += ev[j] < ev[c] || (ev[j] == ev[c] && j < c);
         G[r + (long)rank * n] = V[r + c * P];
-        if (r == 0) eval[(long)u * n + rank] = ev[c];
+        if (r == 0) eval[(long)u * n + rank] = ldexp(ev[c], e);
     }
     if (t == 0) info[u] = done ? 0 : 1;
 }

@@ -90,3 +90,65 @@ def test_dependent_columns_are_refused(hams, cplx):
     st = L.lib().lynx_orthogonalize(H.ctx, L.C128 if cplx else L.F64, L.vptr(X), s.nd, 12, L.MEM_HOST)
     assert st == L.E_CHOLESKY
     assert np.array_equal(X, keep)
+
+
+def narrow_eig(mats):
+    """The library's kernel for narrow_eig on a stack of equal matrices:
+    (vectors, eigenvalues, info), of buffers that held 7 before the call."""
+    from lynx_amd import _lib as L
+    from lynx_amd.hipmem import DeviceArray, synchronize
+    units, n = mats.shape[:2]
+    f = L.lib()._ZN4lynx3gpu10narrow_eigEiPviiPdPiP12ihipStream_t
+    f.restype = None
+    f.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p,
+                  ctypes.c_void_p]
+    M = np.ascontiguousarray(mats.transpose(0, 2, 1))
+    ev, info = np.full((units, n), 7.0), np.full(units, 7, np.int32)
+    d = [DeviceArray.from_numpy(a) for a in (M, ev, info)]
+    f(L.C128 if np.iscomplexobj(M) else L.F64, d[0].ptr, n, units, d[1].ptr, d[2].ptr, None)
+    synchronize()
+    for a, b in zip((M, ev, info), d):
+        b.download(a)
+        b.free()
+    return M.transpose(0, 2, 1), ev, info
+
+
+def hermitian(n, cplx, seed):
+    rng = np.random.default_rng(seed)
+    a = rng.normal(size=(n, n)) + (1j * rng.normal(size=(n, n)) if cplx else 0.0)
+    return a + a.conj().T
+
+
+@pytest.mark.parametrize("n,cplx", [(1, False), (24, False), (33, False), (64, False), (1, True), (12, True),
+                                    (32, True)])
+def test_eigensolve_refuses_values_that_are_not_finite(hams, n, cplx):
+    # one bad value anywhere in the upper triangle: that matrix is refused and
+    # left alone with its eigenvalues, its neighbours are solved
+    good = hermitian(n, cplx, 3)
+    ref = np.linalg.eigvalsh(good)
+    for bad in (np.nan, np.inf, -np.inf) + ((1j * np.inf, complex(0.0, np.nan)) if cplx and n > 1 else ()):
+        for at in {(0, 0), (n - 1, n - 1), (0, n - 1), (n // 2, n - 1)}:
+            if np.iscomplex(bad) and at[0] == at[1]:
+                continue                        # a diagonal's imaginary part is not read
+            mats = np.stack([good, good, good])
+            mats[1][at] = bad
+            keep = mats[1].copy()
+            v, ev, info = narrow_eig(mats)
+            assert list(info) == [0, 1, 0], (bad, at)
+            assert np.array_equal(v[1], keep, equal_nan=True) and np.all(ev[1] == 7.0)
+            for u in (0, 2):
+                assert np.abs(ev[u] - ref).max() < 1e-13 * n * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("n,cplx", [(1, False), (24, False), (64, False), (12, True), (32, True)])
+def test_eigensolve_scales_with_its_matrix(hams, n, cplx):
+    # entries whose squares overflow or vanish: a power of two changes the
+    # eigenvalues by that power and the vectors not at all
+    a = hermitian(n, cplx, 5)
+    v, ev, info = narrow_eig(np.stack([np.ldexp(a.view(float), k).view(a.dtype) for k in (0, 600, 1000, -600, -900)]))
+    assert np.all(info == 0)
+    assert np.abs(a @ v[0] - v[0] * ev[0]).max() < 1e-13 * n * np.abs(ev[0]).max()
+    for i, k in enumerate((0, 600, 1000, -600, -900)):
+        assert np.array_equal(ev[i], np.ldexp(ev[0], k)) and np.array_equal(v[i], v[0]), k
+    v, ev, info = narrow_eig(np.zeros_like(a)[None])
+    assert info[0] == 0 and np.all(ev == 0.0) and np.array_equal(v[0], np.eye(n))
