@@ -206,7 +206,8 @@ lynx_status lynx_chefsi_solve(lynx_ctx *ctx, int dtype, void *psi, int ld, int n
 /* Spectral bounds of H by Lanczos from a glibc srand(seed)/rand() start
  * vector: returns (lambda_min - 0.1, lambda_max * 1.01).  Replaces
  * EigenSolver::lanczos_bounds (EigenSolver.cpp:724-732, Lanczos.hpp:104-198);
- * the reference seeds with 1.  iters (may be NULL) gets the step count. */
+ * the reference seeds with 1.  iters (may be NULL) gets the step count.
+ * LYNX_E_NONFINITE when H yields a NaN or an infinity. */
 lynx_status lynx_lanczos_bounds(lynx_ctx *ctx, int dtype, double *eig_min, double *eig_max,
                                 double tol, int max_iter, unsigned seed, int *iters);
 

@@ -1589,19 +1589,25 @@ lynx_status lynx_lanczos_bounds(lynx_ctx *ctx, int dtype, double *eig_min, doubl
         for (double &x : v) x *= vs;
         HIP_OK(hipMemcpyAsync(vjm1, v.data(), nr * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
         std::vector<double> a(max_iter + 2, 0.0), b(max_iter + 2, 0.0);
+        // a NaN would end the iteration as converged
+        auto finite = [](double v) {
+            if (!std::isfinite(v)) fail(LYNX_E_NONFINITE, "non-finite value in the Lanczos iteration");
+            return v;
+        };
         apply_op(ctx, e, vjm1, n, nullptr, 0, vj, n, 1, 1.0, 0.0, 0.0);
-        a[0] = host_sum(ctx, gpu::dot_partials(e, vjm1, vj, n, ctx->partials.as<double>(), ctx->stream));
+        a[0] = finite(host_sum(ctx, gpu::dot_partials(e, vjm1, vj, n, ctx->partials.as<double>(), ctx->stream)));
         int nb = gpu::lanczos_update(e, vj, vjm1, vjp1, a[0], 0.0, n, ctx->partials.as<double>(), ctx->stream);
-        b[0] = std::sqrt(host_sum(ctx, nb));
+        b[0] = finite(std::sqrt(host_sum(ctx, nb)));
         if (b[0] == 0.0) fail(LYNX_E_UNSUPPORTED, "Lanczos start vector spans an invariant subspace");
         gpu::scale_copy(e, vj, vj, 1.0 / b[0], n, ctx->stream);
         double emin = 0, emax = 0, pmin = 0, pmax = 0, errmin = tol + 1, errmax = tol + 1;
         int j = 0;
         while ((errmin > tol || errmax > tol) && j < max_iter) {
             apply_op(ctx, e, vj, n, nullptr, 0, vjp1, n, 1, 1.0, 0.0, 0.0);
-            a[j + 1] = host_sum(ctx, gpu::dot_partials(e, vj, vjp1, n, ctx->partials.as<double>(), ctx->stream));
+            a[j + 1] =
+                finite(host_sum(ctx, gpu::dot_partials(e, vj, vjp1, n, ctx->partials.as<double>(), ctx->stream)));
             nb = gpu::lanczos_update(e, vjp1, vj, vjm1, a[j + 1], b[j], n, ctx->partials.as<double>(), ctx->stream);
-            b[j + 1] = std::sqrt(host_sum(ctx, nb));
+            b[j + 1] = finite(std::sqrt(host_sum(ctx, nb)));
             if (b[j + 1] == 0.0) break;
             gpu::scale_copy(e, vjp1, vj, 1.0 / b[j + 1], n, ctx->stream);
             const int m = j + 2;
