@@ -244,7 +244,9 @@ lynx_status lynx_psp8_info(const char *path, double *zion, int *lmax, int *lloc,
 /* Timing of the most recent filter call on the context: total and
  * per-kernel-class milliseconds measured with HIP events on its stream.
  * times[0] total, [1] stencil steps, [2] nonlocal gather, [3] nonlocal
- * scatter; launches[0..3] the matching launch counts. */
+ * scatter; launches[0..3] the matching launch counts.  Where no grid point
+ * lies in two spheres, a step's scatter and the next one's gather are one
+ * launch, which counts as a scatter: the gather is then the first step's. */
 lynx_status lynx_last_filter_timing(const lynx_ctx *ctx, double times[4], int launches[4]);
 /* Enable (1) or disable (0) HIP-event timing of filter calls. */
 lynx_status lynx_set_timing(lynx_ctx *ctx, int enable);
@@ -571,9 +573,7 @@ lynx_status lynx_batch_set_graph(lynx_batch *batch, int enable);
  * reference filters in FP64). */
 lynx_status lynx_batch_set_filter_precision(lynx_batch *batch, int precision);
 /* Device time of the last lynx_batch_filter (HIP events around the graph
- * launch or the eager launches) and the number of gather, stencil and scatter
- * kernels it holds (a scatter and the next step's gather in one launch count
- * as two). */
+ * launch or the eager launches) and the number of kernel launches it holds. */
 lynx_status lynx_batch_last_timing(const lynx_batch *batch, double *ms, int *launches);
 /* One CheFSI pass for every unit of the batch: lynx_chefsi_solve on each
  * unit's block psi[u] (device memory, leading dimension ldpsi[u], ncol[u]

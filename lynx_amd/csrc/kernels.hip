@@ -1840,9 +1840,12 @@ void batch_step(BatchPlan *P, int step, int ix, int iold, int iout, bool first, 
 
 int batch_launches(const BatchPlan *P, int steps)
 {
-    int n = (int)(P->sg.size() + 2 * P->ng.size());
-    for (const auto &G : P->ng) n += G.split && G.ngitems > 0;   // the part sums' reduction
-    return n * steps;
+    int n = (int)P->sg.size() * steps;
+    for (const auto &G : P->ng) {
+        if (G.update) n += steps + 1;   // the first gather, steps - 1 updates, the last scatter
+        else n += (G.split ? 3 : 2) * steps;   // split: with the part sums' reduction
+    }
+    return n;
 }
 
 void gram_reduce(int e, const void *work, int nsplit, int n, double alpha, void *C, hipStream_t st)

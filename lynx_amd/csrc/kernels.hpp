@@ -108,8 +108,7 @@ void batch_set_coef(BatchPlan *p, const double *coef, int steps, hipStream_t st)
 // first and last mark the ends of a run of steps, each step taking the output
 // of the one before.
 void batch_step(BatchPlan *P, int step, int ix, int iold, int iout, bool first, bool last, hipStream_t st);
-// Gather, stencil and scatter kernels of a run of steps; a scatter and gather
-// in one launch count as two.
+// Kernel launches of a run of steps.
 int batch_launches(const BatchPlan *P, int steps);
 
 // C (n x n) = alpha * sum of nsplit consecutive n x n partial products in work

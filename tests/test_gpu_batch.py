@@ -2,6 +2,8 @@
 Chebyshev step, replayed from a HIP graph.  Every unit's result is checked
 against the oracle's filter of that unit alone (FP64 1e-11, FP32 2e-5), and
 graph replays against eager launches of the same plan (bitwise)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -119,9 +121,43 @@ def test_graph_replays_match_eager_launches(fcc_kbatch):
         for a, b in zip(yg, ye):
             assert np.array_equal(a, b), rep
     ms, launches = g.last_timing()
-    assert launches == 9 * 3 and ms > 0
+    # nine stencil steps; the spheres share no grid point, so the scatter of a
+    # step and the gather of the next are one launch
+    assert launches == 9 + (9 + 1) and ms > 0
     g.close()
     e.close()
+
+
+@pytest.mark.parametrize("sizes,disjoint,per_step,more", [((), True, 1, 0), ((16, 33), True, 2, 1),
+                                                          ((16, 33), False, 3, 0), ((1025, 40), True, 4, 0)])
+def test_launch_counts(sizes, disjoint, per_step, more):
+    # without projectors; scatter and next gather in one launch; apart (a grid
+    # point in two spheres); apart, with a gather by parts (large spheres).
+    # Alone the gather of large spheres is one launch
+    from lynx_amd import _lib as L, core
+    from test_gpu_nonlocal import N, raw_projectors
+    s = System(N, np.array([6.0, 5.8, 5.5]), np.array([[0.3, 0.4, 0.5]]), with_nonlocal=False)
+    H = s.hamiltonian()
+    if sizes:
+        lat, grid, st, dom, halo = s.core
+        raw = raw_projectors(5, sizes, disjoint, 7, np.sqrt((s.latvec ** 2).sum(axis=1)))[0]
+        H = core.Hamiltonian(0).setup(st, dom, grid, halo, core.NonlocalProjector().setup_raw(**raw))
+    H.set_veff(s.veff)
+    lc, lo, hi = _bounds(0)
+    X = s.random_block(3, 5)
+    for graph in (True, False):
+        bf = core.BatchFilter([(H, None)], graph=graph)
+        for degree in (1, 2, 7):
+            bf.filter([X], degree, lc, lo, hi)
+            assert bf.last_timing()[1] == per_step * degree + more, (graph, degree)
+        bf.close()
+    L.check(L.lib().lynx_set_timing(H.ctx, 1), H.ctx)
+    Y = np.zeros_like(X, order="F")
+    L.check(L.lib().lynx_cheb_filter(H.ctx, L.F64, L.vptr(X), s.nd, L.vptr(Y), s.nd, 3, 7, lc, lo, hi, L.MEM_HOST),
+            H.ctx)
+    ms, n = (ctypes.c_double * 4)(), (ctypes.c_int * 4)()
+    L.check(L.lib().lynx_last_filter_timing(H.ctx, ms, n), H.ctx)
+    assert list(n)[1:] == ([7, 0, 0] if not sizes else [7, 1, 7] if more else [7, 7, 7])
 
 
 def test_batch_errors():
