@@ -68,6 +68,28 @@ def test_bf16_apply_every_vector_shape(n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [(24, 25, 24), (26, 21, 18)])
+def test_bf16_step_rounds_a_float_result_once(n):
+    # the local operator of every vector shape: the nearest bfloat16 value of a
+    # result in float, whatever the order of its sums, and the same bits again.
+    # Half a bfloat16 step, and 80 roundings of 2^-24 of the terms' magnitude
+    from lynx_amd import _lib as L
+    s = System(n, np.array(n) * 0.4275, np.array([[0.3, 0.4, 0.5]]), with_nonlocal=False)
+    op, H = s.oracle_op(), s.hamiltonian()
+    X = s.random_block(3, 47)
+    Xr = np.asfortranarray(from_bf16(to_bf16(X)).reshape(X.shape))
+    ref = op.apply(Xr, s.veff, c=0.1)
+    terms = 0.5 * sum(np.abs(op.arrs[k]).sum() * 2 for k in ("cx", "cy", "cz")) + np.abs(s.veff).max() + 0.1
+    bar = 2.0 ** (np.floor(np.log2(np.abs(ref))) - 8) + 80 * 2.0 ** -24 * terms * np.abs(Xr).max()
+    for shape in [(t, d, z, v) for v in (1, 2, 3) for t in (256, 512) for d in (1, 2) for z in (1, 2, 5)]:
+        L.check(L.lib().lynx_set_stencil_config(H.ctx, *shape), H.ctx)
+        got = apply_bf16(H, X, s.veff, 0.1)
+        assert np.all(np.abs(got - ref) <= bar), shape
+        assert np.array_equal(apply_bf16(H, X, s.veff, 0.1), got), shape
+    L.check(L.lib().lynx_set_stencil_config(H.ctx, 0, 0, 0, 0), H.ctx)
+
+
+@pytest.mark.gpu
 def test_bf16_rejected_where_unsupported():
     from lynx_amd import _lib as L
     s = si8(24)
