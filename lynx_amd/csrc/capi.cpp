@@ -2514,7 +2514,7 @@ lynx_status lynx_batch_solve(lynx_batch *b, int dtype, void *const *psi, const l
             bool aligned = true;
             for (int i = 0; i < 2 * m; ++i) aligned = aligned && reinterpret_cast<uintptr_t>(hp[q.poff + i]) % 16 == 0;
             void *W = b->dgram.get(gpu::narrow_gram_work(dtype, q.N, m, q.nd));
-            gpu::narrow_gram(dtype, {nullptr, 0, A}, lda, {nullptr, 0, B}, ldb, A == B, aligned, q.nd, q.N, m, q.dV, C,
+            gpu::narrow_gram(dtype, {nullptr, A}, lda, {nullptr, B}, ldb, A == B, aligned, q.nd, q.N, m, q.dV, C,
                              W, st);
         };
         // 2. Cholesky-QR per group: S = dV Y^H Y, R^H R = S, psi = Y R^-1 (EigenSolver.cpp:621-641)
@@ -2526,7 +2526,7 @@ lynx_status lynx_batch_solve(lynx_batch *b, int dtype, void *const *psi, const l
                 narrow_gram(q, Yp, q.ldy, Yp, q.ldy, Sg);
                 gpu::narrow_cholesky_inverse(dtype, Sg, N, m, info, st);
                 check_infos(b, info, m, q.units, LYNX_E_CHOLESKY, "Cholesky factorisation of the overlap matrix");
-                gpu::narrow_rotate(dtype, {nullptr, 0, Yp}, q.ldy, {nullptr, 0, Pp}, q.ld, q.nd, N, m, Sg, st);
+                gpu::narrow_rotate(dtype, {nullptr, Yp}, q.ldy, {nullptr, Pp}, q.ld, q.nd, N, m, Sg, st);
                 continue;
             }
             gemm(OC, ON, N, N, (int)q.nd, q.dV, Yp, q.ldy, Yp, q.ldy, Mp, N, m);
@@ -2582,7 +2582,7 @@ lynx_status lynx_batch_solve(lynx_batch *b, int dtype, void *const *psi, const l
                 narrow_gram(q, Pp, q.ld, Yp, q.ldy, Hn);
                 gpu::narrow_eig(dtype, Hn, N, m, D + q.eoff, info, st);
                 check_infos(b, info, m, q.units, LYNX_E_EIG, "subspace eigensolve");
-                gpu::narrow_rotate(dtype, {nullptr, 0, Pp}, q.ld, {nullptr, 0, Pp}, q.ld, q.nd, N, m, Hn, st);
+                gpu::narrow_rotate(dtype, {nullptr, Pp}, q.ld, {nullptr, Pp}, q.ld, q.nd, N, m, Hn, st);
                 continue;
             }
             gemm(OC, ON, N, N, (int)q.nd, q.dV, Pp, q.ld, Yp, q.ldy, Hp, N, m);

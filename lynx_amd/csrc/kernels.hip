@@ -1166,18 +1166,21 @@ template <class S> constexpr int base_rp() { return int(32 / sizeof(S)); }
 // LDS of one workgroup (gfx950: 160 KiB per CU)
 constexpr long kLdsBytes = 160 * 1024;
 
-// rows per band of the non-orthogonal body within the LDS: four planes of
-// pitch * (rows + 2R) + NT elements (two (plane, g-plane) pairs)
-template <class S>
-int nonorth_max_rows(int pitch, int nt)
-{
-    return (int)((kLdsBytes / (4 * (long)sizeof(S)) - nt) / pitch) - 2 * kMaxR;
-}
-
-// LDS pitch of the scalar and non-orthogonal stencil tiles for rows of nx
+// LDS pitch of the scalar stencil tiles for rows of nx
 // points: 64, 128, or 256 for long rows (nx + 2R > 128; 512-thread shapes,
 // with kLongHalo halo slots per thread for up to 256-point rows)
 inline int tile_pitch(int nx) { return nx + 2 * kMaxR <= 64 ? 64 : (nx + 2 * kMaxR <= 128 ? 128 : 256); }
+
+// Whether the one-point-per-thread kernel is offered for rows of nx points in
+// workgroups of nt threads: long rows on 512 threads, and not in complex128
+// skew cells, where a workgroup would hold 114 KB of LDS (one on a CU) and
+// threads whose registers spill.
+template <class S>
+bool point_rows_fit(int nx, int nt, bool orth)
+{
+    if (nx + 2 * kMaxR > 256) return false;
+    return tile_pitch(nx) < 256 || (nt >= 512 && (orth || sizeof(S) <= 8));
+}
 
 // rows per band of the scalar body within the LDS: two planes of
 // pitch * (rows + 2R) + NT elements
@@ -1187,16 +1190,16 @@ int step_max_rows(int pitch, int nt)
     return (int)((kLdsBytes / (2 * (long)sizeof(S)) - nt) / pitch) - 2 * kMaxR;
 }
 
-// Whether rows of nx points fit the scalar / non-orthogonal tiles of NT
+// Whether rows of nx points fit the scalar tiles of NT
 // threads and RP points per thread (row pitch, halo slots, LDS).
 template <class S>
-bool step_rows_fit(int nx, int nt, int rp, bool nonorth)
+bool step_rows_fit(int nx, int nt, int rp)
 {
     const int pitch = tile_pitch(nx);
     if (nx + 2 * kMaxR > 256 || nx > (long)nt * rp) return false;
     const int hb = pitch == 256 ? (nt >= 512 ? kLongHalo : 0) : (nt >= 512 ? 3 : 6);
     if (2 * kMaxR * nx > nt * hb) return false;
-    return (nonorth ? nonorth_max_rows<S>(pitch, nt) : step_max_rows<S>(pitch, nt)) >= 1;
+    return step_max_rows<S>(pitch, nt) >= 1;
 }
 
 template <class S, int RP, int NT>
@@ -1210,7 +1213,7 @@ void launch_step_rp(const StencilGeom &g, const void *x, long ldx, const void *o
     p.ldx = ldx; p.ldo = ldo; p.ldout = ldout;
     p.nx = g.nx; p.ny = g.ny; p.nz = g.nz; p.ncol = ncol;
     const long pts = (long)NT * RP;
-    if (!step_rows_fit<S>(g.nx, NT, RP, false))
+    if (!step_rows_fit<S>(g.nx, NT, RP))
         fail(8, "grid rows longer than the fused stencil kernel's tile are not supported");
     const int pitch = tile_pitch(g.nx);
     const int max_rows = step_max_rows<S>(pitch, NT);
@@ -1310,13 +1313,6 @@ bool launch_step_vec(const StencilGeom &g, const void *x, long ldx, const void *
 }  // namespace
 
 // ------------------------------------------------------------ host wrappers --
-int stencil_points_per_thread(int e, const StepCfg &cfg)
-{
-    int rp = 0;
-    dispatch(e, [&](auto t) { rp = base_rp<decltype(t)>() / std::max(1, cfg.rp_div); });
-    return rp;
-}
-
 bool stencil_shape_fits(int e, int nx, const StepCfg &cfg)
 {
     if (e == B16) {
@@ -1341,7 +1337,7 @@ bool stencil_shape_fits(int e, int nx, const StepCfg &cfg)
                 ok = VW > 0 && lpr <= lanes && 2 * kMaxR * lpr <= nt * hb && nx + 2 * XO <= 128 && nx >= 2 * XO;
             }
         } else {
-            ok = step_rows_fit<S>(nx, nt, base_rp<S>() / std::max(1, cfg.rp_div), false);
+            ok = step_rows_fit<S>(nx, nt, base_rp<S>() / std::max(1, cfg.rp_div));
         }
     });
     return ok;
@@ -1395,30 +1391,27 @@ void stencil_step(int e, const StencilGeom &g, const void *x, long ldx, const vo
     }
     dispatch(e, [&](auto t) {
         using S = decltype(t);
-        constexpr int B = base_rp<S>();
         if constexpr (!Tr<S>::C) {
             if (g.orth && cfg.vec &&
                 launch_vec_modes<S, S>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg, st, coef))
                 return;
         }
         if (!g.orth || Tr<S>::C || tile_pitch(g.nx) < 256) {
-            // one point per thread (stencil_points.hpp); the rows each of the
-            // four shapes takes are those of its tile, points per thread
-            // included, as the tuner lists them.  Real orthogonal rows of
+            // one point per thread (stencil_points.hpp).  Real orthogonal rows of
             // more than 116 points keep the scalar body below, whose threads
             // hold several points: 200 x 40 x 40 x 60 double 183 us against
             // 216 us, bands of two rows beside 12 halo rows; 25 x 27 x 29 x
             // 1600 double takes 209 us here and 311 us there.
             const int nt = cfg.nt >= 512 ? 512 : 256;
-            const int rp = std::max(1, (g.orth ? B : B / 4) / (cfg.rp_div >= 2 ? 2 : 1));
             PointShape sh;
-            if (!step_rows_fit<S>(g.nx, nt, rp, !g.orth) ||
+            if (!point_rows_fit<S>(g.nx, nt, g.orth) ||
                 !point_shape(e, g, cfg.rp_div >= 2 ? nt / 4 * 3 : nt, cfg.nzch, sh))
                 fail(8, "grid rows longer than the fused stencil kernel's tile are not supported");
             points_step(e, g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, sh, st, coef);
             return;
         }
         if constexpr (!Tr<S>::C) {
+            constexpr int B = base_rp<S>();
             if (cfg.nt < 512) fail(8, "grid rows longer than the fused stencil kernel's tile are not supported");
             if (cfg.rp_div >= 2)
                 launch_step_rp<S, B / 2, 512>(g, x, ldx, old, ldo, out, ldout, veff, ncol, a, b, s, cfg.nzch, st, coef);
@@ -1555,7 +1548,7 @@ void build_batch(BatchPlan *P, const BatchUnit *units, int n, hipStream_t st)
         const bool longrow = tile_pitch(g.nx) == 256;
         points[u] = !g.orth || Tr<S>::C || !longrow;
         if (points[u]) {
-            if (!g.orth && longrow && sizeof(S) > 8)
+            if (!point_rows_fit<S>(g.nx, 512, g.orth))
                 fail(8, "complex128 non-orthogonal grids with rows over 116 points are not supported");
             if (!point_shape_batch(P->e, g, shape[u]))
                 fail(8, "grid rows longer than the batched stencil kernel's tile are not supported");

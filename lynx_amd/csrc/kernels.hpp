@@ -48,7 +48,6 @@ struct StepCfg {
 void stencil_step(int e, const StencilGeom &g, const void *x, long ldx, const void *old, long ldo,
                   void *out, long ldout, const void *veff, int ncol, double a, double b, double s,
                   const StepCfg &cfg, hipStream_t st, const void *coef = nullptr);
-int stencil_points_per_thread(int e, const StepCfg &cfg);
 // True when the shape can run the grid's x rows (halo slots and LDS pitch);
 // for vec shapes, also when nx is a multiple of the 16-byte run.
 bool stencil_shape_fits(int e, int nx, const StepCfg &cfg);
@@ -148,14 +147,16 @@ size_t rotate_bf16x3_work(int K, int N);
 void rotate_bf16x3(const float *A, long lda, long M, const double *Q, int ldq, int K, int N, void *C, long ldc,
                    bool c_double, void *work, hipStream_t st);
 // Narrow FP64 / complex128 blocks (kernels_dense.hip): units blocks of equal
-// shape (K rows, n columns), at base + u * stride elements of 8 bytes
-// (complex: 16) or at the addresses of a device table; the n x n matrices of
-// consecutive units are contiguous.  narrow_fits: whether n columns of type e
-// are covered (the limits of the kernels' register tiles and LDS).
+// shape (K rows, n columns), at the addresses of a device table or one at base;
+// the n x n matrices of consecutive units are contiguous.  narrow_fits: whether
+// n columns of type e are covered: as many as the kernels' register tiles and
+// LDS hold, and there they are still ahead of the general ones (30^3 double, us
+// before and now: Cholesky-QR of 33 columns 285 / 108, 48 322 / 153, 64 332 /
+// 233, a pass of 64 with its eigensolve 2263 / 1207; 100^3 x 64 1525 / 908 and
+// 5215 / 2743; complex128 30^3 x 32 1131 / 117 and 3162 / 565).
 constexpr int kNarrowReal = 64, kNarrowComplex = 32;
 struct NarrowBlocks {
     void *base = nullptr;
-    long stride = 0;
     void *const *table = nullptr;
 };
 bool narrow_fits(int e, int n);

@@ -17,15 +17,13 @@ namespace {
 
 typedef double double4v __attribute__((ext_vector_type(4)));
 
-// block u of a batch: entry u of a device pointer table, or base + u * stride
-// elements
+// block u of a batch: entry u of a device pointer table, or the one block
 template <class S>
-__device__ __forceinline__ S *unit_of(const NarrowBlocks &b, long ld, int u)
+__device__ __forceinline__ S *unit_of(const NarrowBlocks &b, int u)
 {
     // (the address space of a pointer read from memory is not known otherwise)
     typedef __attribute__((address_space(1))) S *G;
-    return (S *)(G)reinterpret_cast<unsigned long>(b.table ? static_cast<S *>(b.table[u])
-                                                           : static_cast<S *>(b.base) + (long)u * b.stride);
+    return (S *)(G)reinterpret_cast<unsigned long>(b.table ? b.table[u] : b.base);
 }
 
 // -------------------------------------------------------------------- Gram --
@@ -49,7 +47,7 @@ __global__ void __launch_bounds__(256) k_narrow_gram(NarrowBlocks a, long lda, N
 {
     constexpr int NT = T * (T + 1) / 2, CW = CPLX ? 2 : 1;
     const int u = blockIdx.y;
-    const double *A = unit_of<double>(a, 0, u), *B = SAME ? A : unit_of<double>(b, 0, u);
+    const double *A = unit_of<double>(a, u), *B = SAME ? A : unit_of<double>(b, u);
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     const int lr = l & 15, lk = l >> 4;
     const long len = K * CW;                                   // column length in doubles
@@ -189,8 +187,8 @@ __global__ void __launch_bounds__(256) k_narrow_rotate(NarrowBlocks a, long lda,
         for (int p = 0; p < CW; ++p) sq[p * NP * PQ + j * PQ + k] = in ? Q[((long)j * n + k) * CW + p] : 0.0;
     }
     __syncthreads();
-    const double *A = unit_of<double>(a, 0, u);
-    double *C = unit_of<double>(c, 0, u);
+    const double *A = unit_of<double>(a, u);
+    double *C = unit_of<double>(c, u);
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     const int lr = l & 15, lk = l >> 4;
     const long step = (long)gridDim.x * 64;
@@ -268,7 +266,7 @@ template <> __device__ __forceinline__ Cx from_real<Cx>(double a) { return {a, 0
 // of the factorisation and of the inverse go together: with row k of R known,
 // the trailing part of S loses its outer product and, W holding I times the
 // inverses of the eliminated columns, column j > k of W loses R(k, j) times
-// column k of R^-1.  Two barriers a step; info is the order of the first
+// column k of R^-1.  Three barriers a step; info is the order of the first
 // pivot that is not positive (0: none), as LAPACK's potrf has it.  Bound by
 // the barriers: 22 us at n = 24 real, 10 us for 112 matrices of n = 12
 // complex (potrf and trtri: 64 us in two calls, 29 us).
