@@ -301,21 +301,28 @@ void upload_phases(lynx_ctx *c)
 // A launch has about nx ny ncol lanes per z chunk and the chip holds 256 CUs x
 // 1024 of them.  Where four chunks leave it mostly idle the march along z is
 // what takes the time, and chunks down to three planes (each reads 2R more)
-// are timed too; orthogonal launches with lanes for an eighth of the chip or
-// less have those only, so that the first call stays as short.  Filters of
+// are timed too, or alone where the launch has lanes for an eighth of the chip
+// (skew cells: a 25th) or less, so that the first call stays as short.  Filters of
 // degree 20 and an apply, double: 30^3 x 24 434 -> 297 us, 20^3 x 12 31.8 ->
 // 24 us; at 47 x 45 x 51 x 61 and complex 40^3 x 48 (half and 0.3 of the chip)
-// more than three chunks are slower.
+// more than three chunks are slower.  Skew cells of between a 25th and an
+// eighth of the chip: single precision takes the fine chunks (complex64 24^3 x
+// 24 45 us against 49 us), double and complex128 do not (50^3 x 8, filter of
+// degree 4: 169 and 168 us with and without them, 224 us with them alone), and
+// timing them made the first call longer than it had been (2750 us, 3230 us
+// with them, 2660 us without; 14^3 x 4 715 us, 950 us with all chunks, 560 us
+// with the fine ones alone).
 std::vector<gpu::StepCfg> step_candidates(const lynx_ctx *c, int e, int ncol)
 {
     std::vector<gpu::StepCfg> v;
     const int fill = (int)(256L * 1024 / std::max(1L, (long)c->st.nx * c->st.ny * ncol));
     const int fine = std::min(fill, (c->st.nz + 2) / 3);
+    const int only = c->lat.orth ? 8 : 25;   // fill from which the fine chunks stand alone
     std::vector<int> chunks;
-    if (fill < 8 || fine <= 4 || !c->lat.orth)
+    if (fill < only || fine <= 4)
         for (int nz : {1, 2, 3, 4})
             if (nz == 1 || c->st.nz / nz >= 2 * gpu::kMaxR) chunks.push_back(nz);
-    if (fine > 4) chunks.push_back(fine);
+    if (fine > 4 && (c->lat.orth || fill >= only || gpu::elem_single(e))) chunks.push_back(fine);
     for (int vec : {0, 1, 2, 3})
       for (int align : {0, 1})
         for (int nt : {256, 512})
