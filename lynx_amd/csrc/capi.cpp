@@ -302,7 +302,8 @@ void upload_phases(lynx_ctx *c)
 // 1024 of them.  Where four chunks leave it mostly idle the march along z is
 // what takes the time, and chunks down to three planes (each reads 2R more)
 // are timed too, or alone where the launch has lanes for an eighth of the chip
-// (skew cells: a 25th) or less, so that the first call stays as short.  Filters of
+// (skew cells: a 25th) or less, so that the first call stays as short;
+// orthogonal ones of up to a fifth time them in the place of one chunk.  Filters of
 // degree 20 and an apply, double: 30^3 x 24 434 -> 297 us, 20^3 x 12 31.8 ->
 // 24 us; at 47 x 45 x 51 x 61 and complex 40^3 x 48 (half and 0.3 of the chip)
 // more than three chunks are slower.  Skew cells of between a 25th and an
@@ -321,7 +322,7 @@ std::vector<gpu::StepCfg> step_candidates(const lynx_ctx *c, int e, int ncol)
     std::vector<int> chunks;
     if (fill < only || fine <= 4)
         for (int nz : {1, 2, 3, 4})
-            if (nz == 1 || c->st.nz / nz >= 2 * gpu::kMaxR) chunks.push_back(nz);
+            if (nz == 1 ? !(c->lat.orth && fine > 4) : c->st.nz / nz >= 2 * gpu::kMaxR) chunks.push_back(nz);
     if (fine > 4 && (c->lat.orth || fill >= only || gpu::elem_single(e))) chunks.push_back(fine);
     for (int vec : {0, 1, 2, 3})
       for (int align : {0, 1})
