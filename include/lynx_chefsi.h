@@ -312,8 +312,8 @@ lynx_status lynx_gram(lynx_ctx *ctx, int dtype, const void *a, int lda, const vo
  * n x n matrix q in host memory, FP64 (real dtypes) or complex128 (complex
  * ones), column-major: the rotation of EigenSolver::rotate_orbitals and of
  * the Cholesky step (EigenSolver.cpp:622-641, 674-681), through the product
- * the solve uses for dtype: FP64 / complex128 GEMMs; FP32 GEMMs of q
- * rounded to the block's precision; or, for real FP32 blocks with
+ * the solve uses for dtype: FP64 / complex128 matrix-core kernels up to 64 /
+ * 32 columns, GEMMs above; FP32 GEMMs of q rounded to the block's precision; or, for real FP32 blocks with
  * LYNX_GRAM_BF16X3_ROT, split-BF16x3 matrix-core products of the block and
  * the FP64 q (the reduced-precision pass's rotations under that setting). */
 lynx_status lynx_rotate(lynx_ctx *ctx, int dtype, const void *a, int lda, const double *q, int n, void *c, int ldc,
@@ -344,7 +344,8 @@ lynx_status lynx_get_grid_dims(const lynx_ctx *ctx, int dims[3]);
  * the candidate shapes on the first call for each (grid, dtype, ncol) and
  * caches the fastest (its autotuner; no reference counterpart).
  * lynx_set_stencil_config forces a shape: threads per workgroup 256 or 512,
- * points_div 1 or 2 (points per thread = base / points_div), z_chunks >= 1,
+ * points_div 1 or 2 (points per thread = base / points_div; kernels of one
+ * point per thread: three quarters of the threads), z_chunks >= 1,
  * vector_runs 0..3 (real types: each thread owns 16-byte runs of x points;
  * with 2 the z-direction terms are accumulated forward, with 3 as 2 with
  * loads issued two planes ahead instead of one; adding 4 starts every band

@@ -647,8 +647,10 @@ void gram(lynx_ctx *c, int e, const void *A, long lda, const void *B, long ldb, 
     const bool sym = hermitian || (A == B && lda == ldb);
     if (sym && gpu::narrow_fits(e, n)) {
         // narrow blocks, wherever their kernels' tiles reach: 27,000 x 24 in
-        // 8 us and 12 us for the sum, against 23 us on the 128 x 128 tiles
-        // below and 100 us for the sum of their chunks
+        // 8 us and 12 us for the sum.  At the limit of 64 columns the 96 x 96
+        // tiles below are about as fast: a projection of 64 columns here and of
+        // 66 there 84 and 99 us (30^3), 210 and 214 us (60^3), 689 and 700 us
+        // (100^3)
         const gpu::NarrowBlocks a{const_cast<void *>(A)}, b{const_cast<void *>(B)};
         const bool aligned =
             reinterpret_cast<uintptr_t>(A) % 16 == 0 && reinterpret_cast<uintptr_t>(B) % 16 == 0;
@@ -660,7 +662,7 @@ void gram(lynx_ctx *c, int e, const void *A, long lda, const void *B, long ldb, 
         gpu::gram_f64_fits(static_cast<const double *>(A), lda, static_cast<const double *>(B), ldb)) {
         // a symmetric result (the overlap A^T A, or the projection whose
         // Hermitian part is taken): the hand-written FP64 MFMA kernel forms
-        // only the upper tiles (3.4 against 7.5 ms for rocBLAS's full
+        // only the upper tiles (3.9 against 7.5 ms for rocBLAS's full
         // product at 729,000 x 480); general products stay rocBLAS GEMMs,
         // which run them faster than this kernel
         const int ns = gpu::gram_f64_splits(nd, n);

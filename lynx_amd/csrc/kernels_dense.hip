@@ -40,7 +40,7 @@ __device__ __forceinline__ S *unit_of(const NarrowBlocks &b, int u)
 // complex (297 MB) take 110 us for the overlap and 173 us for the projection
 // (3.4 TB/s of two blocks), where a batched GEMM, which pads the n x n output
 // to 32 x 32 and leaves K in one workgroup, takes 1690 us; 27,000 x 24 real
-// takes 8 and 11 us, in few waves, against 23 us on 128 x 128 tiles.
+// takes 8 and 11 us, in few waves.
 template <bool CPLX, int T, bool SAME>
 __global__ void __launch_bounds__(256) k_narrow_gram(NarrowBlocks a, long lda, NarrowBlocks b, long ldb, long K,
                                                      int n, long kch, int vec, double *__restrict__ part)

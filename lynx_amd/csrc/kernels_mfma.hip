@@ -231,8 +231,8 @@ __global__ void __launch_bounds__(kThreads) k_gram_bf16x3(const float *__restric
 // lanes (16 columns, two k) read distinct banks.  32-deep blocks need more
 // registers than three workgroups per CU leave.
 //
-// Bound by the matrix cores: 480 columns of 90^3 points 3.4 ms (50 TFLOP/s of
-// the half product), with 128 x 128 tiles and 32-deep blocks, one workgroup
+// Bound by the matrix cores: 480 columns of 90^3 points 3.8 to 4.0 ms (42 to 44
+// TFLOP/s of the half product), with 128 x 128 tiles and 32-deep blocks, one workgroup
 // per CU, 5.9 ms (5.4 ms A = B); 160 of 60^3 0.22 ms.  Fragments straight from
 // memory, without LDS or barriers: 5.2-5.6 ms.
 constexpr int kDT = 96;           // C tile edge
@@ -367,7 +367,7 @@ __global__ void __launch_bounds__(256, 3) k_gram_f64(const double *__restrict__ 
 // from L1 and L2.
 //
 // Bound by the matrix cores and the refill at the strips' ends: 90^3 x 480
-// 3.7 ms (50 TFLOP/s of the half product; 2.4 ms at the rate of a large
+// 3.8 ms (44 TFLOP/s of the half product; 2.4 ms at the rate of a large
 // library GEMM), where a library GEMM with the explicit inverse took 5.5 ms
 // and the copy back 0.95 ms; 60^3 x 160 0.22 ms (0.43 ms), 30^3 x 65 19 us
 // (30 us).  32 points per wave, at three waves per SIMD: 4.3 ms.
@@ -702,12 +702,14 @@ int gram_f64_splits(long K, int N)
     const int tiles = (N + kDT - 1) / kDT;
     const int pairs = tiles * (tiles + 1) / 2;
     // one round of the three workgroups that a CU holds: 780 items in 768
-    // slots took 4.4 ms, 765 take 3.4 ms (480 columns of 90^3 points)
+    // slots took 4.4 ms, 765 take 3.8 ms (480 columns of 90^3 points)
     constexpr long kSlots = 768;
     const long most = (K + kDKB - 1) / kDKB;
     long best = std::max(1L, std::min(kSlots / pairs, most));
     // wide blocks, whose tiles alone half fill the last round, are split as
-    // far as that fills it, the partial products within a quarter of a block
+    // far as that fills it, the partial products within a quarter of a block:
+    // the projection of 2700 columns of 40^3 points 15.6 ms in one split, 14.4
+    // ms in five
     auto fill = [&](long s) { return (double)(pairs * s) / (double)((pairs * s + kSlots - 1) / kSlots * kSlots); };
     for (long s = best + 1; s <= std::min({8L, most, K / (4L * N)}); ++s)
         if (fill(s) > 1.05 * fill(best)) best = s;
